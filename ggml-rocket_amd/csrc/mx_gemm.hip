@@ -13,11 +13,13 @@
 //   dequant_f16   a weight panel -> fp16 [rows][K] (the resident-fp16 form, "prepacked-q").
 //   pack_weight   a ggml Q8_0 / Q6_K / MXFP4 payload -> its split HBM layout (mx_weights.h).
 //
-// Three GEMM kernels: a register-staged one that decodes any weight format into LDS
-// (gemm_kernel), for fp16 weights one that moves both operands into LDS by DMA (gemm_f16_kernel,
-// and its two-width variant gemm_f16_cols_kernel), and for M <= 128 one that decodes the weight
-// straight into MFMA operands (gemm_skinny_kernel). The launcher picks a kernel and tile
-// configuration per call from the output shape.
+// The GEMM kernels: a register-staged one that decodes any weight format into LDS (gemm_kernel);
+// for fp16 weights two that move both operands into LDS by DMA, gemm_f16_1w_kernel for tiled
+// weights and gemm_f16_kernel (with its two-width variant gemm_f16_cols_kernel) for row-major
+// ones; for Q4_K and Q8_0 one that moves every operand by DMA and decodes from LDS
+// (gemm_q4k_kernel); and for M <= 128 one that decodes the weight straight into MFMA operands
+// (gemm_skinny_kernel). The launcher picks a kernel and tile configuration per call from the
+// output shape.
 
 #include <algorithm>
 #include <cmath>
@@ -786,7 +788,7 @@ struct ColsTile {
     int N, n0, m0;
 };
 
-template <class C, int TNW, int COL0, bool TL>
+template <class C, int TNW, int COL0>
 __device__ __forceinline__ void cols_body(const uint16_t * __restrict__ Ap, const float * __restrict__ scales,
                                           int64_t lda, int M, int K, ColsTile tb, uint8_t * smem, int wm) {
     constexpr int DK = C::RB / 2, NS = C::NSTAGES, NJ = TNW / 32;
@@ -808,7 +810,7 @@ __device__ __forceinline__ void cols_body(const uint16_t * __restrict__ Ap, cons
         const int slot = (q * C::NW + wave) * WAVE + lane;
         const int r = slot / C::CH, c = (slot % C::CH) ^ ((r / C::RPW) & (C::CH - 1));
         const int64_t row = min(m0 + r, M - 1), k = 8 * c;
-        asrc[q] = Ap + (TL ? tiled_index(row, k, K) : row * lda + k);
+        asrc[q] = Ap + row * lda + k;
     }
 #pragma unroll
     for (int q = 0; q < PB; q++) {
@@ -818,21 +820,21 @@ __device__ __forceinline__ void cols_body(const uint16_t * __restrict__ Ap, cons
             const int slot = (q * 4 + wm) * WAVE + lane;
             const int r = slot / C::CH, c = (slot % C::CH) ^ ((r / C::RPW) & (C::CH - 1));
             const int64_t row = row0 + min(n0 + COL0 + r, N - 1), k = 8 * c;
-            bsrc[q] = W + (TL ? tiled_index(row, k, K) : row * K + k);
+            bsrc[q] = W + row * K + k;
         } else {
             // instruction q * 8 + wave of the whole B tile (rows of both columns in order; the
             // swizzle is the same, since BN0 is a multiple of 16)
             const int slot = min(q * C::NW + wave, C::NBI - 1) * WAVE + lane;
             const int r = slot / C::CH, c = (slot % C::CH) ^ ((r / C::RPW) & (C::CH - 1));
             const int64_t row = row0 + min(n0 + r, N - 1), k = 8 * c;
-            bsrc[q] = W + (TL ? tiled_index(row, k, K) : row * K + k);
+            bsrc[q] = W + row * K + k;
         }
     }
     const int wave_s = __builtin_amdgcn_readfirstlane(wave), wm_s = __builtin_amdgcn_readfirstlane(wm);
     auto issue = [&](int s) {
         uint8_t * st = smem + (s % NS) * C::STAGE;
         s = min(s, nk - 1);
-        const int64_t off = (int64_t)s * (TL ? DK * 16 : DK);
+        const int64_t off = (int64_t)s * DK;
 #pragma unroll
         for (int q = 0; q < C::PA; q++) dma16(asrc[q] + off, st + (q * C::NW + wave_s) * 1024);
 #pragma unroll
@@ -926,7 +928,7 @@ __device__ __forceinline__ void cols_body(const uint16_t * __restrict__ Ap, cons
     }
 }
 
-template <int BM, int BN0, int BN1, int DK, int NS, bool TL>
+template <int BM, int BN0, int BN1, int DK, int NS>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_f16_cols_kernel(GemmArgs args) {
     using C = ColsCfg<BM, BN0, BN1, DK, NS>;
@@ -946,14 +948,220 @@ gemm_f16_cols_kernel(GemmArgs args) {
         }
     tb.n0 = (nt - ntb) * C::BN;
     tb.m0 = mt * C::BM;
-    if (wave / 4 == 0) cols_body<C, BN0, 0, TL>(args.A, args.scales, args.lda, args.M, args.K, tb, smem, wave % 4);
-    else cols_body<C, BN1, BN0, TL>(args.A, args.scales, args.lda, args.M, args.K, tb, smem, wave % 4);
+    if (wave / 4 == 0) cols_body<C, BN0, 0>(args.A, args.scales, args.lda, args.M, args.K, tb, smem, wave % 4);
+    else cols_body<C, BN1, BN0>(args.A, args.scales, args.lda, args.M, args.K, tb, smem, wave % 4);
 }
 
-// Zero the outputs of a split-K launch (a fill kernel rather than a memset, so the launch
-// sequence stays capturable).
-// Zeroes the outputs a split-K launch adds into: one block per (row, weight group), 16-byte
-// stores where the row start allows them.
+// ---------------------------------------------------------------------------------------------
+// Tiled fp16 weights (T_F16T): one wave per SIMD, every memory instruction under an MFMA
+//
+// What bounds a tile of gemm_f16_kernel above is the CU's LDS and the instruction order, not the
+// MFMAs: eight waves of 64 x 128 read 96 bytes of LDS a clock at the full MFMA rate beside the 32
+// the DMA writes (128 is the CU's limit), and all of them issue their reads and DMA in one burst
+// after each stage's barrier. Here a block is four waves, one per SIMD, so a wave has 512 registers
+// and takes up to 128 x 112 of the output (accumulators in AGPRs): a 256 x 224 tile reads 69 bytes
+// a clock. With no second wave to cover for it, the wave has to keep its own MFMAs issuing: stage
+// s is multiplied from registers while stage s + 1's fragments are read and stage s + NS's DMA is
+// issued, one read or one DMA after each MFMA (a 16 x 16 x 32 MFMA takes 16 clocks, a read or a
+// DMA 4 to 8 of issue). Two things keep those gaps that short: buffer loads, whose source is a
+// fixed lane offset plus one scalar stage offset (global loads took a scalar chain and a 64-bit
+// vector add each: 119 us instead of 107 at 512 x 28672 x 4096), and the empty asm statements at the
+// stage's end, which hold the accumulators in AGPRs across the loop (left alone, the compiler moves
+// them through VGPRs: hundreds of moves a stage).
+//
+// A stage is 32 values of K for the tile's BM + BN rows; LDS slot (row r, chunk p) of its 4 chunks a
+// row holds logical chunk p ^ ((r / 4) & 3), so the 16 rows of a fragment read fall on 16 distinct
+// bank groups. Per stage, after its first MFMA (whose operands are the wave's last reads of the
+// stage's buffer): wait until stage s + 1 has landed (the (NS - 2) stages behind it may be in
+// flight), one barrier, then buffer s % NS is refilled with stage s + NS. Past the last stage the
+// last one is fetched again into buffers nobody reads, so the wait counts are constants.
+// Rows past M or N read the last real row. The MFMA's first operand is the weight, so a lane holds
+// 4 consecutive output columns of one row and stores 16 bytes at once.
+//
+// A launch of few tiles splits K args.ksplit ways (each split a slab of args.part, summed in split
+// order by reduce_splits_kernel). Measured against gemm_f16_kernel and its two-width variant on
+// cold weights, one box, M x N x K (us): 512 x 28672 x 4096 118.2 -> 102.6, 2048 x 6144 x 4096 101.1 ->
+// 85.6, 2048 x 3072 x 8192 121.2 -> 93.7, 512 x 4096 x 14336 83.1 -> 69 (split 4), 512 x 4096 x 4096
+// 29.9 -> 24.2, 48 x 1536 x 8960 30.8 -> 13.1 (split 8); over 95 shapes 1.2x (M 48-2048).
+// ---------------------------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// D(16x16, f32) += A(16x32, f16) . B(32x16, f16). Lane l holds A row and B column l % 16, K slots
+// 8 (l / 16) + 0..7; D: column l % 16, rows 4 (l / 16) + 0..3.
+__device__ __forceinline__ void mfma16(const half8 & a, const half8 & b, f32x4 & c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+template <int BM_, int BN_, int WGM_, int WGN_, int NS_>
+struct OneWaveCfg {
+    static constexpr int BM = BM_, BN = BN_, NS = NS_, NW = 4, THREADS = 256, WGN = WGN_;
+    static constexpr int TM = BM / WGM_, TN = BN / WGN_, MI = TM / 16, NJ = TN / 16;
+    static constexpr int RB = 64;                                   // bytes of a row's 32 values
+    // DMA instructions per wave and stage, 4 KB of LDS a block each; a BN of 96, 160 or 224 ends
+    // half-way through one, whose other half fetches rows nobody reads into the stage's padding
+    static constexpr int PA = (BM * RB + 4095) / 4096, PB = (BN * RB + 4095) / 4096, PER = PA + PB;
+    static constexpr int A_BYTES = PA * 4096, STAGE = A_BYTES + PB * 4096, LDS = NS * STAGE;
+    static_assert(WGM_ * WGN_ == 4 && TM % 16 == 0 && TN % 16 == 0, "wave tile");
+    static_assert(LDS <= 160 * 1024 && NS >= 3 && (NS - 1) * PER <= 63, "ring");
+};
+
+template <int BM, int BN, int WGM, int WGN, int NS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+gemm_f16_1w_kernel(GemmArgs args) {
+#ifdef __HIP_DEVICE_COMPILE__   // the buffer resource type exists in the device pass only
+    using C = OneWaveCfg<BM, BN, WGM, WGN, NS>;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int t = threadIdx.x, lane = t % WAVE, wave = __builtin_amdgcn_readfirstlane(t / WAVE);
+    const int wm = wave / WGN, wn = wave % WGN;
+    const int ks = args.ksplit > 1 ? args.ksplit : 1;
+    int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int split = tile % ks;
+    tile /= ks;
+    const int mt = tile % args.m_tiles, nt = tile / args.m_tiles;
+    int g = 0;
+    const uint16_t * W = (const uint16_t *)args.g[0].W;
+    int64_t row0 = args.g[0].row0;
+    int N = args.g[0].N, ntb = args.g[0].ntile_begin;
+    float * Cp = args.g[0].C;
+    int64_t ldc = args.g[0].ldc;
+#pragma unroll
+    for (int i = 1; i < GEMM_MAX_GROUPS; i++)
+        if (i < args.ng && nt >= args.g[i].ntile_begin) {
+            g = i;
+            W = (const uint16_t *)args.g[i].W; row0 = args.g[i].row0; N = args.g[i].N;
+            ntb = args.g[i].ntile_begin; Cp = args.g[i].C; ldc = args.g[i].ldc;
+        }
+    split_target(args, g, split, Cp, ldc);
+    const int n0 = (nt - ntb) * BN, m0 = mt * BM;
+    const int M = args.M, K = args.K, nk_all = K / 32;
+    const int per = (nk_all + ks - 1) / ks, kb = split * per;
+    const int nk = max(0, min(nk_all, kb + per) - kb);
+
+    // each operand's buffer starts at the tile's first 16-row block; a lane's offset in it stays
+    // below 16 * K * 32 bytes (the launcher keeps K under ONE_WAVE_MAX_K)
+    constexpr int KSTEP = 1024;   // bytes of a row block one stage of K takes
+    const int64_t a0 = tiled_index(m0, 0, K), b0 = tiled_index((row0 + n0) & ~(int64_t)15, 0, K);
+    const char * abase = (const char *)(args.A + a0) + (int64_t)kb * KSTEP;
+    const char * bbase = (const char *)(W + b0) + (int64_t)kb * KSTEP;
+    int aoff[C::PA], boff[C::PB];
+#pragma unroll
+    for (int q = 0; q < C::PA; q++) {
+        const int slot = (q * 4 + wave) * WAVE + lane, r = slot / 4, c = (slot % 4) ^ ((r / 4) & 3);
+        const int64_t row = min(m0 + r, M - 1);
+        aoff[q] = (int)(2 * (tiled_index(row, 8 * c, K) - a0));
+    }
+#pragma unroll
+    for (int q = 0; q < C::PB; q++) {
+        const int slot = (q * 4 + wave) * WAVE + lane, r = slot / 4, c = (slot % 4) ^ ((r / 4) & 3);
+        const int64_t row = row0 + min(n0 + r, N - 1);
+        boff[q] = (int)(2 * (tiled_index(row, 8 * c, K) - b0));
+    }
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void *)abase, 0, 0x7FFFFFFF, 0x00020000);
+    const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc((void *)bbase, 0, 0x7FFFFFFF, 0x00020000);
+    auto issue1 = [&](uint8_t * st, int soff, int q) {
+        if (q < C::PA)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ar, (lptr_t)(st + wave * 1024 + q * 4096), 16, aoff[q], soff, 0, 0);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(br, (lptr_t)(st + wave * 1024 + q * 4096), 16, boff[q - C::PA], soff, 0, 0);
+    };
+    const int lr = lane % 16, lg = lane / 16;
+    const int co = (lg ^ ((lr / 4) & 3)) * 16;
+    const int a_off = (wm * C::TM + lr) * 64 + co, b_off = C::A_BYTES + (wn * C::TN + lr) * 64 + co;
+
+    f32x4 acc[C::MI][C::NJ];
+#pragma unroll
+    for (int i = 0; i < C::MI; i++)
+#pragma unroll
+        for (int j = 0; j < C::NJ; j++) acc[i][j] = f32x4{0, 0, 0, 0};
+
+    struct Frags {
+        half8 a[C::MI], b[C::NJ];
+    };
+    auto read1 = [&](const uint8_t * st, Frags & f, int r) {
+        if (r < C::NJ) f.b[r] = *(const half8 *)(st + b_off + r * 1024);
+        else f.a[r - C::NJ] = *(const half8 *)(st + a_off + (r - C::NJ) * 1024);
+    };
+    constexpr int NR = C::MI + C::NJ, NM = C::MI * C::NJ;
+    int buf = 0;                                   // byte offset of the stage being multiplied
+    const int last = (nk - 1) * KSTEP;
+    int soff = min(NS * KSTEP, last);              // source offset of the stage NS ahead
+    auto stage = [&](const Frags & F, Frags & G) {
+        const int nbuf = buf == (NS - 1) * C::STAGE ? 0 : buf + C::STAGE;
+        const uint8_t * st = smem + nbuf;
+        uint8_t * fill = smem + buf;
+#pragma unroll
+        for (int p = 0; p < NM; p++) {
+            const int i = p / C::NJ, j = p % C::NJ;
+            mfma16(F.b[j], F.a[i], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (p == 0) {   // stage s + 1 has landed, and every wave is done with this stage's buffer
+                wait_vm_lgkm0<(NS - 2) * C::PER>();
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            constexpr int RS = NM >= 3 * NR ? 2 : 1;
+            if (p >= 1 && (p - 1) % RS == 0 && (p - 1) / RS < NR) {
+                read1(st, G, (p - 1) / RS);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            constexpr int DS = (NM - 2) / C::PER > 0 ? (NM - 2) / C::PER : 1;
+            if (p >= 2 && (p - 2) % DS == 0 && (p - 2) / DS < C::PER) {
+                issue1(fill, soff, (p - 2) / DS);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        static_assert((NR - 1) * (NM >= 3 * NR ? 2 : 1) + 1 < NM && C::PER <= NM - 2, "a slot for every read and DMA");
+        // the accumulators stay in AGPRs from stage to stage
+#pragma unroll
+        for (int i = 0; i < C::MI; i++)
+#pragma unroll
+            for (int j = 0; j < C::NJ; j++) asm volatile("" : "+a"(acc[i][j]));
+        buf = nbuf;
+        soff = min(soff + KSTEP, last);
+    };
+    if (nk > 0) {
+        Frags f0, f1;
+#pragma unroll
+        for (int p = 0; p < NS; p++)
+#pragma unroll
+            for (int q = 0; q < C::PER; q++) issue1(smem + p * C::STAGE, min(p * KSTEP, last), q);
+        wait_vm_lgkm0<(NS - 1) * C::PER>();
+        __builtin_amdgcn_s_barrier();
+#pragma unroll
+        for (int r = 0; r < NR; r++) read1(smem, f0, r);
+        int s = 0;
+        for (; s + 2 <= nk; s += 2) {
+            stage(f0, f1);
+            stage(f1, f0);
+        }
+        if (s < nk) stage(f0, f1);
+        wait_vm_lgkm0<0>();
+    }
+    // epilogue: the lane holds output row lr of each 16-row block, columns 4 lg .. 4 lg + 3 of each
+    // 16-column one. Every scale is loaded before the first store (loads and stores retire in order).
+    float sc[C::MI];
+#pragma unroll
+    for (int i = 0; i < C::MI; i++) sc[i] = args.scales[min(m0 + wm * C::TM + i * 16 + lr, M - 1)];
+    const bool vec = ((reinterpret_cast<uintptr_t>(Cp) | (uintptr_t)(4 * ldc)) & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < C::MI; i++) {
+        const int r = m0 + wm * C::TM + i * 16 + lr;
+        if (r >= M) continue;
+        float * crow = Cp + (int64_t)r * ldc;
+#pragma unroll
+        for (int j = 0; j < C::NJ; j++) {
+            const int n = n0 + wn * C::TN + j * 16 + 4 * lg;
+            const f32x4 v = acc[i][j] * sc[i];
+            if (n >= N) continue;
+            if (vec) *(f32x4 *)(crow + n) = v;
+            else
+#pragma unroll
+                for (int e = 0; e < 4; e++) crow[n + e] = v[e];
+        }
+        __builtin_amdgcn_sched_barrier(0);   // one row block's products at a time: no spills
+    }
+#endif
+}
+
 // ---------------------------------------------------------------------------------------------
 // Q4_K GEMM with every operand by LDS DMA (the per-call dequant route for Q4_K weights).
 //
@@ -1557,6 +1765,9 @@ __global__ void __launch_bounds__(256) reduce_splits_kernel(GemmArgs a, int ks) 
     }
 }
 
+// Zeroes the outputs a split-K launch adds into (a fill kernel rather than a memset, so the launch
+// sequence stays capturable): one block per (row, weight group), 16-byte stores where the row
+// start allows them.
 __global__ void __launch_bounds__(256) zero_rows_kernel(GemmArgs args) {
     const GemmGroup & G = args.g[blockIdx.y];
     float * row = G.C + (int64_t)blockIdx.x * G.ldc;
@@ -1709,10 +1920,12 @@ hipError_t launch_pack_act_tiled(const float * X, int64_t ldx, int M, int K, uin
 // Tile configurations. The launcher picks one per call (choose_cfg); MI355X_GEMM_CFG=<id>
 // forces one (for tuning and for the tests, which run every configuration).
 //   0-3  register-staged kernel with the weight decoded into LDS: every weight type.
-//   4-15 LDS-DMA kernel: fp16 weights only (row-major or tiled); 15 has wave columns of two
-//        widths (gemm_f16_cols_kernel), 21 and 22 are that tile with 32-deep stages, three or
-//        four of them in flight where 15 has one of 64 (the 256 x 224 tile's DMA waits are
-//        what bounds it); 23 and 24 are 8 and 14 with eight 32-deep stages.
+//   4-15 LDS-DMA kernel: row-major fp16 weights; 15 has wave columns of two widths
+//        (gemm_f16_cols_kernel), 21 and 22 are that tile with 32-deep stages, three or four of
+//        them in flight where 15 has one of 64 (the 256 x 224 tile's DMA waits are what bounds
+//        it); 23 and 24 are 8 and 14 with eight 32-deep stages. Of these only 8, 9, 10 and 23
+//        also take tiled weights, where 25-34 cannot split K (see choose_cfg).
+//   25-34 one wave per SIMD (gemm_f16_1w_kernel): tiled fp16 weights, any K split.
 //   16-19 Q4_K with every operand by DMA (gemm_q4k_kernel), K % 256 == 0; 18 and 19 split K
 //        (q4k_split). 20 is the skinny kernel's id (use_skinny), not a tile configuration.
 // choose_cfg prices a launch from two rates: a block's own pace, rounds * (ov_us + MFMA work
@@ -1721,14 +1934,17 @@ hipError_t launch_pack_act_tiled(const float * X, int64_t ldx, int M, int K, uin
 // / bw (bigger tiles fetch less per FLOP but keep fewer bytes in flight per CU). The two
 // overlap, so the estimate is their 4-norm (pace^4 + feed^4)^(1/4), which follows the measured
 // transition between the regimes better than the max; a split-K launch adds zc microseconds per
-// MB of output (the zero fill and the second addend's atomics). The four were fitted per
-// configuration to measurements on tiled weights at M = 128-2048, N = 1024-28672,
-// K = 2880-14336, each launch on a weight panel no earlier launch left in the caches: mean
-// error 2-9% per configuration, and over 50 shapes the chosen configurations cost 0.6% more
-// than the best measured ones.
-enum CfgKind { REG = 0, DMA = 1, Q4KDMA = 2, NONE = 3 };
+// MB of output (the zero fill and the second addend's atomics), or for 25-34 the reduction's
+// launch and its slabs (ONEW_RED_US + ONEW_RED_US_MB per MB of partials). The four were fitted per
+// configuration to measurements on tiled weights, each launch on a weight panel no earlier launch
+// left in the caches: 4-24 at M = 128-2048, N = 1024-28672, K = 2880-14336, mean error 2-9% per
+// configuration, and over 50 shapes the chosen configurations cost 0.6% more than the best
+// measured ones; 25-34 at M = 48-2048, N = 1024-28672, K = 2048-14336 with splits of 1-8, mean error
+// 4-10%, and over 95 shapes the choices cost 1.5% more than the best of all configurations.
+enum CfgKind { REG = 0, DMA = 1, Q4KDMA = 2, NONE = 3, ONEW = 4 };
 struct CfgDesc {
-    int kind;        // REG: gemm_kernel, DMA: gemm_f16_kernel / _cols, Q4KDMA: gemm_q4k_kernel
+    int kind;        // REG: gemm_kernel, DMA: gemm_f16_kernel / _cols, Q4KDMA: gemm_q4k_kernel,
+                     // ONEW: gemm_f16_1w_kernel
     int bm, bn, ksplit;
     int dk;          // K per LDS stage (0 for the register-staged kernel)
     double tf_cu;    // TFLOP/s per CU
@@ -1762,6 +1978,16 @@ static constexpr CfgDesc kCfgs[] = {
     {DMA, 256, 224, 1, 32, 6.78, 10.1, 8.73, 0.00},   // 22: as 15, 5 stages of 32
     {DMA, 128, 128, 2, 32, 3.59, 0.0, 17.89, 1.65},   // 23: as 8, 8 stages of 32
     {DMA, 64, 128, 1, 32, 2.70, 1.4, 17.12, 0.00},    // 24: as 14, 8 stages of 32
+    {ONEW, 256, 224, 1, 32, 7.98, 8.86, 10.36, 0.00},  // 25: tiled weights, 4 waves of 128x112, 5 stages of 32
+    {ONEW, 256, 192, 1, 32, 7.79, 7.09, 11.10, 0.00},  // 26: 128x96, 5 stages
+    {ONEW, 256, 160, 1, 32, 7.38, 6.43, 11.92, 0.00},  // 27: 128x80, 5 stages
+    {ONEW, 256, 128, 1, 32, 6.65, 5.42, 13.21, 0.00},  // 28: 128x64, 6 stages
+    {ONEW, 128, 224, 1, 32, 6.44, 6.08, 12.43, 0.00},  // 29: 64x112, 6 stages
+    {ONEW, 128, 192, 1, 32, 6.22, 5.35, 13.47, 0.00},  // 30: 64x96, 7 stages
+    {ONEW, 128, 128, 1, 32, 5.70, 4.78, 14.32, 0.00},  // 31: 64x64, 9 stages
+    {ONEW, 128, 96, 1, 32, 4.66, 3.69, 14.63, 0.00},   // 32: 64x48, 9 stages
+    {ONEW, 128, 64, 1, 32, 4.11, 3.31, 17.89, 0.00},   // 33: 64x32, 9 stages
+    {ONEW, 64, 128, 1, 32, 4.14, 4.19, 15.82, 0.00},   // 34: 32x64, 9 stages
 };
 constexpr int FIRST_DMA_CFG = 4;
 constexpr int N_CFGS = sizeof(kCfgs) / sizeof(kCfgs[0]);
@@ -1794,10 +2020,24 @@ static hipError_t launch_f16(const GemmArgs & a, int nblocks, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <int BM, int BN0, int BN1, int DK, int NS, bool TL>
+template <int BM, int BN0, int BN1, int DK, int NS>
 static hipError_t launch_cols(const GemmArgs & a, int nblocks, hipStream_t st) {
     using C = ColsCfg<BM, BN0, BN1, DK, NS>;
-    auto kern = gemm_f16_cols_kernel<BM, BN0, BN1, DK, NS, TL>;
+    auto kern = gemm_f16_cols_kernel<BM, BN0, BN1, DK, NS>;
+    static bool attr = false;
+    if (!attr) {
+        hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    hipLaunchKernelGGL(kern, dim3(nblocks), dim3(C::THREADS), C::LDS, st, a);
+    return hipGetLastError();
+}
+
+template <int BM, int BN, int WGM, int WGN, int NS>
+static hipError_t launch_1w(const GemmArgs & a, int nblocks, hipStream_t st) {
+    using C = OneWaveCfg<BM, BN, WGM, WGN, NS>;
+    auto kern = gemm_f16_1w_kernel<BM, BN, WGM, WGN, NS>;
     static bool attr = false;
     if (!attr) {
         hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
@@ -1822,25 +2062,46 @@ static hipError_t launch_q4k(const GemmArgs & a, int nblocks, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <bool TL>
-static hipError_t launch_dma_cfg(int cfg, const GemmArgs & a, int nblocks, hipStream_t st) {
+// row-major fp16 weights
+static hipError_t launch_row_cfg(int cfg, const GemmArgs & a, int nblocks, hipStream_t st) {
     switch (cfg) {
-        case 15: return launch_cols<256, 128, 96, 64, 2, TL>(a, nblocks, st);
-        case 21: return launch_cols<256, 128, 96, 32, 4, TL>(a, nblocks, st);
-        case 22: return launch_cols<256, 128, 96, 32, 5, TL>(a, nblocks, st);
-        case 23: return launch_f16<128, 128, 4, 2, 32, 8, 2, TL>(a, nblocks, st);
-        case 24: return launch_f16<64, 128, 2, 2, 32, 8, 1, TL>(a, nblocks, st);
-        case 4: return launch_f16<256, 256, 4, 2, 64, 2, 1, TL>(a, nblocks, st);
-        case 5: return launch_f16<128, 128, 4, 2, 64, 4, 1, TL>(a, nblocks, st);
-        case 6: return launch_f16<64, 128, 2, 2, 128, 3, 1, TL>(a, nblocks, st);
-        case 7: return launch_f16<128, 64, 2, 2, 128, 3, 1, TL>(a, nblocks, st);
-        case 8: return launch_f16<128, 128, 4, 2, 64, 4, 2, TL>(a, nblocks, st);
-        case 9: return launch_f16<64, 128, 2, 2, 128, 3, 2, TL>(a, nblocks, st);
-        case 10: return launch_f16<128, 128, 4, 2, 32, 4, 1, TL>(a, nblocks, st);
-        case 11: return launch_f16<128, 128, 4, 2, 32, 8, 1, TL>(a, nblocks, st);
-        case 12: return launch_f16<256, 128, 4, 2, 64, 3, 1, TL>(a, nblocks, st);
-        case 13: return launch_f16<128, 256, 2, 4, 64, 3, 1, TL>(a, nblocks, st);
-        case 14: return launch_f16<64, 128, 2, 2, 64, 6, 1, TL>(a, nblocks, st);
+        case 15: return launch_cols<256, 128, 96, 64, 2>(a, nblocks, st);
+        case 21: return launch_cols<256, 128, 96, 32, 4>(a, nblocks, st);
+        case 22: return launch_cols<256, 128, 96, 32, 5>(a, nblocks, st);
+        case 23: return launch_f16<128, 128, 4, 2, 32, 8, 2, false>(a, nblocks, st);
+        case 24: return launch_f16<64, 128, 2, 2, 32, 8, 1, false>(a, nblocks, st);
+        case 4: return launch_f16<256, 256, 4, 2, 64, 2, 1, false>(a, nblocks, st);
+        case 5: return launch_f16<128, 128, 4, 2, 64, 4, 1, false>(a, nblocks, st);
+        case 6: return launch_f16<64, 128, 2, 2, 128, 3, 1, false>(a, nblocks, st);
+        case 7: return launch_f16<128, 64, 2, 2, 128, 3, 1, false>(a, nblocks, st);
+        case 8: return launch_f16<128, 128, 4, 2, 64, 4, 2, false>(a, nblocks, st);
+        case 9: return launch_f16<64, 128, 2, 2, 128, 3, 2, false>(a, nblocks, st);
+        case 10: return launch_f16<128, 128, 4, 2, 32, 4, 1, false>(a, nblocks, st);
+        case 11: return launch_f16<128, 128, 4, 2, 32, 8, 1, false>(a, nblocks, st);
+        case 12: return launch_f16<256, 128, 4, 2, 64, 3, 1, false>(a, nblocks, st);
+        case 13: return launch_f16<128, 256, 2, 4, 64, 3, 1, false>(a, nblocks, st);
+        case 14: return launch_f16<64, 128, 2, 2, 64, 6, 1, false>(a, nblocks, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+// tiled fp16 weights
+static hipError_t launch_tiled_cfg(int cfg, const GemmArgs & a, int nblocks, hipStream_t st) {
+    switch (cfg) {
+        case 8: return launch_f16<128, 128, 4, 2, 64, 4, 2, true>(a, nblocks, st);
+        case 9: return launch_f16<64, 128, 2, 2, 128, 3, 2, true>(a, nblocks, st);
+        case 10: return launch_f16<128, 128, 4, 2, 32, 4, 1, true>(a, nblocks, st);
+        case 23: return launch_f16<128, 128, 4, 2, 32, 8, 2, true>(a, nblocks, st);
+        case 25: return launch_1w<256, 224, 2, 2, 5>(a, nblocks, st);
+        case 26: return launch_1w<256, 192, 2, 2, 5>(a, nblocks, st);
+        case 27: return launch_1w<256, 160, 2, 2, 5>(a, nblocks, st);
+        case 28: return launch_1w<256, 128, 2, 2, 6>(a, nblocks, st);
+        case 29: return launch_1w<128, 224, 2, 2, 6>(a, nblocks, st);
+        case 30: return launch_1w<128, 192, 2, 2, 7>(a, nblocks, st);
+        case 31: return launch_1w<128, 128, 2, 2, 9>(a, nblocks, st);
+        case 32: return launch_1w<128, 96, 2, 2, 9>(a, nblocks, st);
+        case 33: return launch_1w<128, 64, 2, 2, 9>(a, nblocks, st);
+        case 34: return launch_1w<64, 128, 2, 2, 9>(a, nblocks, st);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1863,11 +2124,8 @@ static hipError_t launch_cfg(int cfg, const GemmArgs & a, int nblocks, hipStream
             return hipErrorInvalidValue;
         }
     }
-    if (kCfgs[cfg].kind == DMA) {
-        if (WT != T_F16 && WT != T_F16T) return hipErrorInvalidValue;
-        return launch_dma_cfg<WT == T_F16T>(cfg, a, nblocks, st);
-    }
-    if constexpr (WT == T_F16T) return hipErrorInvalidValue;
+    if constexpr (WT == T_F16T) return launch_tiled_cfg(cfg, a, nblocks, st);
+    else if (kCfgs[cfg].kind == DMA) return WT == T_F16 ? launch_row_cfg(cfg, a, nblocks, st) : hipErrorInvalidValue;
     else switch (cfg) {
         case 0: return launch_one<WT, 128, 128, 2, 2, 2, 1>(a, nblocks, st);
         case 1: return launch_one<WT, 128, 128, 2, 2, 2, 0>(a, nblocks, st);   // split a.ksplit ways
@@ -1934,17 +2192,63 @@ static int q4k_split(const GemmArgs & a, int bm, int bn, int cap) {
     return (nsb + per - 1) / per;
 }
 
+// gemm_f16_1w_kernel addresses a tile's rows by 32-bit byte offsets (16 row blocks of 32 K bytes)
+constexpr int ONE_WAVE_MAX_K = 1 << 21;
+
 static bool cfg_fits(int c, int wt, int K) {
     const CfgDesc & d = kCfgs[c];
     if (d.kind == NONE) return false;
     if (d.kind == REG) return wt != T_F16T;
     if (d.kind == Q4KDMA) return (wt == T_Q4_K || (wt == T_Q8_0 && d.bm == 128)) && K % 256 == 0;
+    if (d.kind == ONEW) return wt == T_F16T && K % d.dk == 0 && K <= ONE_WAVE_MAX_K;
+    if (wt == T_F16T && c != 8 && c != 9 && c != 10 && c != 23) return false;
     if ((wt != T_F16 && wt != T_F16T) || K % d.dk) return false;
     return d.ksplit == 1 || K / d.dk >= 2;
 }
 
-// fp16 weights: the DMA configuration with the least estimated time (the CfgDesc model; every
-// DMA block has a CU to itself, so a launch runs in ceil(blocks / CUs) rounds).
+// A configuration's estimated microseconds with a K split (the CfgDesc model), and for the one-wave
+// kernel the reduction of its split: a launch, and its slabs written and read back.
+constexpr double ONEW_RED_US = 4.65, ONEW_RED_US_MB = 0.335;
+// `tiles`: the launch's output tiles, out_mb: its output; an estimate known to pass `limit` (from
+// its larger term) is returned as the limit, without the roots.
+static double cfg_estimate(const CfgDesc & d, int K, int tiles, double out_mb, int ks, int cus, double limit) {
+    const int blocks = tiles * ks;
+    const int rounds = (blocks + cus - 1) / cus;
+    const double kb = (double)K / ks;
+    const double pace = rounds * (d.ov_us + 2.0 * d.bm * d.bn * kb / (d.tf_cu * 1e6));
+    const double feed = (double)blocks * (d.bm + d.bn) * kb * 2.0 / (d.bw * 1e6);
+    const double split = ks == 1 ? 0.0 : d.kind == ONEW ? ONEW_RED_US + ONEW_RED_US_MB * ks * out_mb : d.zc * out_mb;
+    if (std::max(pace, feed) + split >= limit) return limit;
+    const double p2 = pace * pace, f2 = feed * feed;
+    return std::sqrt(std::sqrt(p2 * p2 + f2 * f2)) + split;
+}
+
+// Tiled fp16 weights: the one-wave configuration and K split with the least estimate, among the
+// splits whose partials fit (`slabs` of them) and that leave a split at least 512 values of K (16
+// stages; shorter ones are mostly pipeline fill). Without room for two slabs the two-way atomic
+// splits of the older kernel compete too: a deep K over few tiles is still faster split (512 x
+// 4096 x 14336 83 us against 91 unsplit). K past ONE_WAVE_MAX_K: the older kernel alone.
+static void choose_tiled(const GemmArgs & a, int slabs, int & cfg, int & ks) {
+    const int cus = cu_count();
+    const double out_mb = (double)a.M * (double)tiles_n_cols(a) * 4.0 / 1e6;
+    double best = 1e30;
+    cfg = 10;
+    ks = 1;
+    for (int c = FIRST_DMA_CFG; c < N_CFGS; c++) {
+        const CfgDesc & d = kCfgs[c];
+        if (!cfg_fits(c, T_F16T, a.K)) continue;
+        if (d.kind == DMA && slabs >= 2 && a.K <= ONE_WAVE_MAX_K) continue;
+        const int tiles = tiles_of(a, d.bm, d.bn);
+        for (int s : {1, 2, 3, 4, 6, 8}) {
+            if (d.kind == DMA ? s != d.ksplit : s > 1 && (s > slabs || a.K / s < 512)) continue;
+            const double us = cfg_estimate(d, a.K, tiles, out_mb, s, cus, best);
+            if (us < best - 1e-9) { best = us; cfg = c; ks = s; }
+        }
+    }
+}
+
+// Row-major fp16 weights: the DMA configuration with the least estimated time (the CfgDesc model;
+// every DMA block has a CU to itself, so a launch runs in ceil(blocks / CUs) rounds).
 // Q4_K weights (K % 256 == 0): the all-DMA kernel where it fills the chip (below).
 // Other weights: split K when the output is skinny for its depth (reg_split), otherwise the
 // unsplit register-staged tile with the best grid fill times its relative per-CU efficiency
@@ -1957,25 +2261,19 @@ static int choose_cfg(int wt, const GemmArgs & a) {
         }
     }
     const int cus = cu_count();
-    if (wt == T_F16 || wt == T_F16T) {
+    if (wt == T_F16) {
         int best = -1;
-        double best_us = 0.0;
+        double best_us = 1e30;
+        const double out_mb = (double)a.M * (double)tiles_n_cols(a) * 4.0 / 1e6;
         for (int c = FIRST_DMA_CFG; c < N_CFGS; c++) {
             if (kCfgs[c].kind != DMA || !cfg_fits(c, wt, a.K)) continue;
             const CfgDesc & d = kCfgs[c];
             // the model was fitted on tiled weights; on row-major ones a 32-deep stage reads half
             // cache lines per row (qkv at M 512: 496 against 613 TFLOP/s for 64-deep stages), so
             // it is left to the K % 64 != 0 shapes that nothing else takes
-            if (wt == T_F16 && d.dk == 32 && a.K % 64 == 0) continue;
-            const int blocks = tiles_of(a, d.bm, d.bn) * d.ksplit;
-            const int rounds = (blocks + cus - 1) / cus;
-            const double kb = (double)a.K / d.ksplit;
-            const double pace = rounds * (d.ov_us + 2.0 * d.bm * d.bn * kb / (d.tf_cu * 1e6));
-            const double feed = (double)blocks * (d.bm + d.bn) * kb * 2.0 / (d.bw * 1e6);
-            const double p2 = pace * pace, f2 = feed * feed;
-            double us = std::sqrt(std::sqrt(p2 * p2 + f2 * f2));
-            if (d.ksplit > 1) us += d.zc * (double)a.M * tiles_n_cols(a) * 4.0 / 1e6;
-            if (best < 0 || us < best_us - 1e-9) { best = c; best_us = us; }
+            if (d.dk == 32 && a.K % 64 == 0) continue;
+            const double us = cfg_estimate(d, a.K, tiles_of(a, d.bm, d.bn), out_mb, d.ksplit, cus, best_us);
+            if (us < best_us - 1e-9) { best = c; best_us = us; }
         }
         if (best >= 0) return best;
     }
@@ -2131,13 +2429,14 @@ static hipError_t launch_skinny(const GemmArgs & a, int nblocks, int gpb, hipStr
     return hipGetLastError();
 }
 
-// A launch's configuration and K split. The split is at most `cap` ways: the number of partial
-// slabs [M][sum of N] the caller's workspace holds, and at least 2.
+// A launch's configuration and K split. A split past two ways takes a slab of the caller's
+// workspace per way; the one-wave kernel's always does.
 struct GemmPlan {
     bool skinny;
-    int cfg;    // kCfgs index (unused for the skinny kernel)
-    int ks;     // K split
-    int gpb;    // skinny kernel: K groups per block
+    int cfg;      // kCfgs index (unused for the skinny kernel)
+    int ks;       // K split
+    int gpb;      // skinny kernel: K groups per block
+    bool slabs;   // each split writes its slab of the partials (else two ways, added into the output)
 };
 
 static int64_t total_cols(const GemmArgs & a) {
@@ -2146,14 +2445,29 @@ static int64_t total_cols(const GemmArgs & a) {
     return n;
 }
 
-static int split_cap(const GemmArgs & a, size_t part_bytes) {
+// partial slabs [M][sum of N] the workspace holds, at most 64
+static int split_slabs(const GemmArgs & a, size_t part_bytes) {
     const size_t slab = (size_t)a.M * (size_t)total_cols(a) * sizeof(float);
-    const size_t n = slab ? part_bytes / slab : 0;
-    return (int)std::max<size_t>(2, std::min<size_t>(n, 64));
+    return (int)std::min<size_t>(slab ? part_bytes / slab : 0, 64);
 }
 
-static GemmPlan plan_gemm(int wt, const GemmArgs & a, int cap) {
+static GemmPlan plan_gemm(int wt, const GemmArgs & a, int slabs) {
     GemmPlan p{};
+    const int cap = std::max(slabs, 2);   // two ways need no slab: they add into the output
+    if (wt == T_F16T) {
+        const char * e = getenv("MI355X_GEMM_CFG");
+        const int forced = (e && *e) ? atoi(e) : -1;
+        if (forced >= 0 && forced < N_CFGS && cfg_fits(forced, wt, a.K)) {
+            p.cfg = forced;
+            p.ks = kCfgs[forced].ksplit;
+            if (const char * k = getenv("MI355X_GEMM_KSPLIT"))
+                if (kCfgs[forced].kind == ONEW) p.ks = std::min(std::max(atoi(k), 1), std::max(slabs, 1));
+        } else {
+            choose_tiled(a, slabs, p.cfg, p.ks);
+        }
+        p.slabs = kCfgs[p.cfg].kind == ONEW && p.ks > 1;
+        return p;
+    }
     if (use_skinny(wt, a)) {
         p.skinny = true;
         p.cfg = SKINNY_CFG;
@@ -2161,12 +2475,14 @@ static GemmPlan plan_gemm(int wt, const GemmArgs & a, int cap) {
         const int ch = skinny_chunk_depth(wt, a);
         const int ngroups = ((a.K + 63) / 64 + ch - 1) / ch;
         p.ks = (ngroups + p.gpb - 1) / p.gpb;
+        p.slabs = p.ks > 2;
         return p;
     }
     p.cfg = choose_cfg(wt, a);
     const CfgDesc & d = kCfgs[p.cfg];
     p.ks = p.cfg == 1 ? reg_split(a, cap)
          : (d.kind == Q4KDMA && d.ksplit > 1) ? q4k_split(a, d.bm, d.bn, cap) : d.ksplit;
+    p.slabs = p.ks > 2;
     return p;
 }
 
@@ -2185,17 +2501,18 @@ bool q8_0_decode_first(int64_t M, int64_t N, int64_t K) {
 
 size_t gemm_split_bytes(int wt, const GemmArgs & a) {
     const GemmPlan p = plan_gemm(wt, a, 64);
-    return p.ks > 2 ? (size_t)p.ks * (size_t)a.M * (size_t)total_cols(a) * sizeof(float) : 0;
+    return p.slabs ? (size_t)p.ks * (size_t)a.M * (size_t)total_cols(a) * sizeof(float) : 0;
 }
 
 bool gemm_accumulates(int wt, const GemmArgs & a, size_t part_bytes) {
-    return plan_gemm(wt, a, split_cap(a, part_bytes)).ks == 2;
+    const GemmPlan p = plan_gemm(wt, a, split_slabs(a, part_bytes));
+    return p.ks == 2 && !p.slabs;
 }
 
 hipError_t launch_gemm(int wt, const GemmArgs & a_in, int /*unused*/, hipStream_t st, bool c_zeroed, float * part,
                        size_t part_bytes) {
     GemmArgs a = a_in;
-    const GemmPlan p = plan_gemm(wt, a, part ? split_cap(a, part_bytes) : 2);
+    const GemmPlan p = plan_gemm(wt, a, part ? split_slabs(a, part_bytes) : 0);
     const int bn = p.skinny ? 32 * SK_NW : kCfgs[p.cfg].bn;
     int nt = 0;
     int64_t pcol = 0;
@@ -2207,11 +2524,11 @@ hipError_t launch_gemm(int wt, const GemmArgs & a_in, int /*unused*/, hipStream_
     }
     a.m_tiles = p.skinny ? 1 : (a.M + kCfgs[p.cfg].bm - 1) / kCfgs[p.cfg].bm;
     a.ksplit = p.ks;
-    a.part = p.ks > 2 ? part : nullptr;
+    a.part = p.slabs ? part : nullptr;
     a.ldp = pcol;
     const int nblocks = nt * a.m_tiles * a.ksplit;
     if (nblocks <= 0) return hipSuccess;
-    if (p.ks == 2 && !c_zeroed) {
+    if (p.ks == 2 && !p.slabs && !c_zeroed) {
         hipLaunchKernelGGL(zero_rows_kernel, dim3(a.M, a.ng), dim3(256), 0, st, a);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;

@@ -586,3 +586,44 @@ def test_pack_clear_then_accumulating_gemm(mx):
     assert np.array_equal(outs[0], outs[1])
     rows = np.arange(0, M, 16)
     _assert_bars(O.mul_mat(O.F16, W16, Xf[rows], N, K), outs[1][rows], len(rows), N, "pack-clear + zeroed GEMM")
+
+
+# The one-wave-per-SIMD kernel of tiled weights: every tile, with 1 to 8 K splits, an odd and an
+# even number of 32-value stages (one fewer than the ring holds, and splits of unequal length), M
+# and N off every tile, two members of one panel (the second at a row that is no multiple of 16),
+# and an output whose rows are not 16-byte aligned.
+@pytest.mark.parametrize("K,ksplit", [(96, 1), (1312, 1), (1312, 3), (4096, 8)])
+@pytest.mark.parametrize("cfg", range(25, 35))
+def test_one_wave_gemm(mx, monkeypatch, cfg, K, ksplit):
+    import torch
+    monkeypatch.setenv("MI355X_GEMM_CFG", str(cfg))
+    monkeypatch.setenv("MI355X_GEMM_KSPLIT", str(ksplit))
+    M, Ns, rows = 275, (240, 176), 240 + 8 + 176
+    Xf = O.fill_normal((M, K), 1500 + K)
+    W16 = O.f32_to_f16_bits(O.fill_normal((rows, K), 1501 + K, 0.0, 0.02))
+    Wp = np.zeros((rows, -(-K // 64) * 64), dtype=np.uint16)   # tile_f16 takes whole 64-value slabs
+    Wp[:, :K] = W16
+    if K % 64:   # the tiled layout holds K % 32 == 0: build it here, tile by tile
+        t = np.zeros((-(-rows // 16) * 16, K), dtype=np.uint16)
+        t[:rows] = W16
+        t = t.reshape(-1, 16, K // 32, 32).transpose(0, 2, 1, 3)
+        w = torch.from_numpy(np.ascontiguousarray(t).view(np.uint8).reshape(-1)).cuda()
+    else:
+        w = mx.tile_f16(O.F16, mx.upload_weight(O.F16, Wp, rows, K), rows, K)
+    a16, sc = mx.pack_act(_dev(Xf), tiled=True)
+    part = torch.empty(ksplit * M * sum(Ns) * 4, dtype=torch.uint8, device="cuda")
+    got = []
+    for _ in range(2):
+        cs = [torch.full((M, N + 1 + 3 * i), float("nan"), dtype=torch.float32, device="cuda") for i, N in enumerate(Ns)]
+        arr = (mx.GemmOut * 2)()
+        for i, (N, row0) in enumerate(zip(Ns, (0, 248))):
+            arr[i] = mx.GemmOut(w.data_ptr(), rows, row0, N, cs[i].data_ptr(), cs[i].stride(0))
+        mx.check(mx.lib().mi355x_gemm_ws(F16_T, mx._ptr(a16), mx._ptr(sc), M, K, arr, 2, mx._ptr(part), part.numel(), 0,
+                                         mx.stream_handle()), "gemm_ws")
+        torch.cuda.synchronize()
+        got.append([c.cpu().numpy() for c in cs])
+    for i, (N, row0) in enumerate(zip(Ns, (0, 248))):
+        assert np.array_equal(got[0][i][:, :N], got[1][i][:, :N]), "launches differ"
+        assert np.isnan(got[0][i][:, N:]).all(), "wrote past N"
+        ref = O.mul_mat(O.F16, W16[row0:row0 + N], Xf, N, K)
+        _assert_bars(ref, got[0][i][:, :N], M, N, f"one-wave cfg {cfg} K={K} split {ksplit}")
