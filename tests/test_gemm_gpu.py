@@ -627,3 +627,23 @@ def test_one_wave_gemm(mx, monkeypatch, cfg, K, ksplit):
         assert np.isnan(got[0][i][:, N:]).all(), "wrote past N"
         ref = O.mul_mat(O.F16, W16[row0:row0 + N], Xf, N, K)
         _assert_bars(ref, got[0][i][:, :N], M, N, f"one-wave cfg {cfg} K={K} split {ksplit}")
+
+
+@pytest.mark.parametrize("wtype", [O.F16, O.Q8_0, O.Q4_0, O.Q4_K, O.Q5_K, O.Q6_K, O.MXFP4])
+@pytest.mark.parametrize("rows,K", [(17, 64), (1, 576), (33, 1344)])
+def test_f16_tiled_ragged(mx, wtype, rows, K):
+    """The tiled decode takes 16 rows x 512 K a block and 128 K a wave: rows and K that end inside
+    them, against the row-major decode's values, bit for bit; nothing is written past the layout."""
+    import torch
+    if wtype in SUPER_BLOCK:
+        K = (K + 255) // 256 * 256
+    W = O.fill_normal((rows, K), 1600 + wtype, 0.0, 0.02)
+    w = mx.upload_weight(wtype, O.f32_to_f16_bits(W) if wtype == O.F16 else O.quantize(wtype, W), rows, K)
+    want = mx.dequant_f16(wtype, w, rows, K).view(torch.int16)
+    rp = (rows + 15) // 16 * 16
+    out = torch.full((rp * K + 512,), -1, dtype=torch.int16, device="cuda")
+    mx.check(mx.lib().mi355x_weight_f16_tiled(wtype, mx._ptr(w), rows, K, mx._ptr(out), mx.stream_handle()), "tiled")
+    torch.cuda.synchronize()
+    assert bool((out[rp * K:] == -1).all())
+    got = out[:rp * K].view(rp // 16, K // 32, 16, 32).permute(0, 2, 1, 3).reshape(rp, K)[:rows]
+    assert bool((got == want).all())
