@@ -251,24 +251,61 @@ static size_t mul_mat_part_offset(int64_t M, int64_t K) {
     return (mi355x_mul_mat_workspace(M, K) + 255) & ~(size_t)255;
 }
 
-// Weights of the register-staged decode kernel run faster at M >= 512 decoded once per call into
-// tiled fp16 (one pass over the weight) and multiplied by the fp16 GEMM than decoded inside the
-// GEMM, where the decode sits on every tile's load path. Measured per call on MI355X with cold
-// weights over N, K in {3072, 4096, 8192, 14336}: Q6_K, Q5_K and MXFP4 1.06-1.48x at M 512 and
-// 1.24-1.91x at M 2048; Q8_0 and Q4_0 1.08-1.15x at M 512 with N >= K, 0.92-0.99x with N < K (the
-// fp16 GEMM's few output tiles there), 1.19-1.52x at M 2048. Not M 128 and below (the decode pass
-// costs more than the GEMM saves). Q4_K's all-DMA decode kernel is 0.83-1.38x of the two-pass
-// form depending on the shape: the two-pass form wins where N >= K and the fp16 weight is at most
-// 64 MB (1.02-1.38x, e.g. 1.20x for N 6144, K 4096 at M 512), and loses on larger panels, whose
-// fp16 form no longer stays in the 256 MB last-level cache (0.83x for N 28672, K 4096 at M 512).
-// Q8_0 with whole 256-value blocks has an all-DMA kernel of its own, which wins at M < 1024 but
-// on one kind of shape (mx::q8_0_decode_first). Same fp16 weights and activations either way.
+static int device_cus() {
+    static int cus = 0;   // read once: this may run while a stream is being captured
+    if (cus == 0) {
+        int dev = 0;
+        hipDeviceProp_t p;
+        cus = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess &&
+               p.multiProcessorCount > 0) ? p.multiProcessorCount : 256;
+    }
+    return cus;
+}
+
+// The share of the chip that an all-DMA launch of bm x 256 tiles keeps busy over its rounds.
+static double tile_fill(int64_t M, int64_t N, int bm) {
+    const int64_t t = ((M + bm - 1) / bm) * ((N + 255) / 256), cus = device_cus();
+    return (double)t / (double)((t + cus - 1) / cus * cus);
+}
+
+// Where a weight decoded once per call into tiled fp16 (one pass over the weight, at HBM rate) and
+// multiplied by the one-wave fp16 GEMM is faster than decoded inside the GEMM. Measured per call on
+// MI355X with cold weights over N, K in {1024, 2048, 3072, 4096, 6144, 8192, 14336, 28672} and M 65-2048
+// (in-GEMM time over decode-first time); never at M <= 128, where the skinny kernels win 1.1-2.5x.
+//   Q6_K, Q5_K, MXFP4, Q4_0 (register-staged decode kernel): 1.1-2.3x from M 384 on; below that up to
+//     2^25 weights, 0.95-1.5x, on larger panels 0.82-1.05x (MXFP4, its slowest in-GEMM decode, 1.15-1.4x
+//     up to 2^26).
+//   Q4_K and Q8_0 (all-DMA decode kernels):
+//     up to 2^25 weights 0.95-1.7x from M 129 on, except that past 2^23 weights a K of 2 N or more is split
+//     inside the all-DMA kernel, which is as fast (0.85-1.03x) up to M 767, and loses 1.1-1.6x beyond;
+//     larger panels: from M 768 (Q8_0) or 1024 (Q4_K) on 1.0-1.5x. Below that the all-DMA kernel wins
+//     where its tiles fill the chip (14336 x 4096 at M 512, 224 tiles: 0.93x) and loses 1.1-1.4x where
+//     the last round is mostly empty (at M 600, 280 tiles); Q8_0 past 2^26 weights, whose decode pass
+//     moves twice the bytes, only from M 768.
+// Panels under 2^22 weights keep lines drawn with the older fp16 GEMM: such calls are a few
+// microseconds of launches either way. Same fp16 weights and activations in both forms.
 static bool mul_mat_decode_first(int wtype, int64_t M, int64_t N, int64_t K) {
-    if (K % 64 || M < 512) return false;
-    if (wtype == mx::T_Q6_K || wtype == mx::T_Q5_K || wtype == mx::T_MXFP4) return true;
-    if (wtype == mx::T_Q4_K) return N >= K && N * K <= ((int64_t)1 << 25);
-    if (wtype == mx::T_Q8_0) return mx::q8_0_decode_first(M, N, K);
-    return wtype == mx::T_Q4_0 && (N >= K || M >= 1024);
+    if (K % 64 || M <= 128) return false;
+    const int64_t w = N * K;
+    const bool panel = w >= ((int64_t)1 << 22), w25 = w <= ((int64_t)1 << 25), w26 = w <= ((int64_t)1 << 26);
+    const bool split = K >= 2 * N && w > ((int64_t)1 << 23);
+    switch (wtype) {
+        case mx::T_Q6_K:
+        case mx::T_Q5_K: return M >= 512 || (panel && (M >= 384 || w25));
+        case mx::T_MXFP4: return M >= 512 || (panel && (M >= 384 || w26));
+        case mx::T_Q4_0: return (panel && (M >= 384 || w25)) || (M >= 512 && (N >= K || M >= 1024));
+        case mx::T_Q4_K:
+            if (!panel) return M >= 512 && N >= K;
+            if (split) return M >= 768;
+            if (w25 || M >= 1024) return true;
+            return M >= 384 && std::max(tile_fill(M, N, 128), tile_fill(M, N, 256)) < 0.8;
+        case mx::T_Q8_0:
+            if (!panel) return M >= 1024 || (M >= 512 && K % 256 && N >= K);
+            if (split) return M >= 768;
+            if (w25 || M >= 768) return true;
+            return M >= 384 && w26 && tile_fill(M, N, 128) < 0.8;
+        default: return false;
+    }
 }
 
 MI355X_API int mi355x_mul_mat_decode_first(int wtype, int64_t M, int64_t N, int64_t K) {
@@ -422,17 +459,6 @@ static FaLayout fa_layout(const mx::FaArgs & f) {
     L.pml = L.po + (f.nsplit > 1 ? align256(rows * f.DV * 4) : 0);
     L.total = L.pml + (f.nsplit > 1 ? align256(rows * 8) : 0);
     return L;
-}
-
-static int device_cus() {
-    static int cus = 0;   // read once: this may run while a stream is being captured
-    if (cus == 0) {
-        int dev = 0;
-        hipDeviceProp_t p;
-        cus = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess &&
-               p.multiProcessorCount > 0) ? p.multiProcessorCount : 256;
-    }
-    return cus;
 }
 
 // The launch of an op: wave tasks per block and KV split (nsplit_req > 0: that split). One block

@@ -2517,19 +2517,6 @@ static GemmPlan plan_gemm(int wt, const GemmArgs & a, int slabs) {
     return p;
 }
 
-// Q8_0 at M < 1024 with whole 256-value blocks runs the all-DMA kernel (choose_cfg) faster than
-// the decode-first form (the whole weight decoded to tiled fp16, then the fp16 GEMM) except where
-// N >= K, the weight has more than 2^24 values and its 128 x 256 tiles leave more than 30% of the
-// chip idle (8192 x 3072 at M 512: 71.2 against 66.0 us); at M >= 1024 the decode-first form is
-// as fast or faster (its weight decoded once, against once per 128-row M tile), e.g. 14336 x 4096
-// at M 2048: 296 against 366 us.
-bool q8_0_decode_first(int64_t M, int64_t N, int64_t K) {
-    if (M >= 1024) return true;
-    if (K % 256) return N >= K;
-    const int64_t tiles = ((M + 127) / 128) * ((N + 255) / 256);
-    return N >= K && N * K > ((int64_t)1 << 24) && tiles < (cu_count() * 7 + 9) / 10;
-}
-
 size_t gemm_split_bytes(int wt, const GemmArgs & a) {
     const GemmPlan p = plan_gemm(wt, a, 64);
     return p.slabs ? (size_t)p.ks * (size_t)a.M * (size_t)total_cols(a) * sizeof(float) : 0;

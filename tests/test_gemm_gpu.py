@@ -647,3 +647,13 @@ def test_f16_tiled_ragged(mx, wtype, rows, K):
     assert bool((out[rp * K:] == -1).all())
     got = out[:rp * K].view(rp // 16, K // 32, 16, 32).permute(0, 2, 1, 3).reshape(rp, K)[:rows]
     assert bool((got == want).all())
+
+
+@pytest.mark.parametrize("wtype,M,N,K", [(O.Q4_K, 129, 2064, 2048), (O.Q8_0, 131, 2048, 2112), (O.Q4_0, 129, 2176, 1984),
+                                         (O.Q6_K, 130, 4112, 1024), (O.MXFP4, 129, 1040, 4096)])
+def test_mul_mat_decode_first_from_129_rows(mx, wtype, M, N, K):
+    """The decode-first form at its fewest rows and smallest panels, against the in-GEMM decode and
+    the oracle; at 128 rows the skinny kernel runs."""
+    assert mx.lib().mi355x_mul_mat_decode_first(wtype, M, N, K) == 1
+    assert mx.lib().mi355x_mul_mat_decode_first(wtype, 128, N, K) == 0
+    test_mul_mat_decode_first(mx, wtype, M, N, K)
