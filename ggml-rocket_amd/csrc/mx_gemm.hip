@@ -1956,7 +1956,7 @@ hipError_t launch_pack_act_tiled(const float * X, int64_t ldx, int M, int K, uin
 //        them in flight where 15 has one of 64 (the 256 x 224 tile's DMA waits are what bounds
 //        it); 23 and 24 are 8 and 14 with eight 32-deep stages. Of these only 8, 9, 10 and 23
 //        also take tiled weights, where 25-34 cannot split K (see choose_cfg).
-//   25-34 one wave per SIMD (gemm_f16_1w_kernel): tiled fp16 weights, any K split.
+//   25-35 one wave per SIMD (gemm_f16_1w_kernel): tiled fp16 weights, any K split.
 //   16-19 Q4_K with every operand by DMA (gemm_q4k_kernel), K % 256 == 0; 18 and 19 split K
 //        (q4k_split). 20 is the skinny kernel's id (use_skinny), not a tile configuration.
 // choose_cfg prices a launch from two rates: a block's own pace, rounds * (ov_us + MFMA work
@@ -1965,12 +1965,12 @@ hipError_t launch_pack_act_tiled(const float * X, int64_t ldx, int M, int K, uin
 // / bw (bigger tiles fetch less per FLOP but keep fewer bytes in flight per CU). The two
 // overlap, so the estimate is their 4-norm (pace^4 + feed^4)^(1/4), which follows the measured
 // transition between the regimes better than the max; a split-K launch adds zc microseconds per
-// MB of output (the zero fill and the second addend's atomics), or for 25-34 the reduction's
+// MB of output (the zero fill and the second addend's atomics), or for 25-35 the reduction's
 // launch and its slabs (ONEW_RED_US + ONEW_RED_US_MB per MB of partials). The four were fitted per
 // configuration to measurements on tiled weights, each launch on a weight panel no earlier launch
 // left in the caches: 4-24 at M = 128-2048, N = 1024-28672, K = 2880-14336, mean error 2-9% per
 // configuration, and over 50 shapes the chosen configurations cost 0.6% more than the best
-// measured ones; 25-34 at M = 48-2048, N = 1024-28672, K = 2048-14336 with splits of 1-8, mean error
+// measured ones; 25-35 at M = 48-2048, N = 1024-28672, K = 2048-14336 with splits of 1-8, mean error
 // 4-10%, and over 95 shapes the choices cost 1.5% more than the best of all configurations.
 enum CfgKind { REG = 0, DMA = 1, Q4KDMA = 2, NONE = 3, ONEW = 4 };
 struct CfgDesc {
@@ -2019,6 +2019,7 @@ static constexpr CfgDesc kCfgs[] = {
     {ONEW, 128, 96, 1, 32, 4.66, 3.69, 14.63, 0.00},   // 32: 64x48, 9 stages
     {ONEW, 128, 64, 1, 32, 4.11, 3.31, 17.89, 0.00},   // 33: 64x32, 9 stages
     {ONEW, 64, 128, 1, 32, 4.14, 4.19, 15.82, 0.00},   // 34: 32x64, 9 stages
+    {ONEW, 256, 256, 1, 32, 7.98, 10.5, 9.50, 0.00},   // 35: 128x128, 5 stages
 };
 constexpr int FIRST_DMA_CFG = 4;
 constexpr int N_CFGS = sizeof(kCfgs) / sizeof(kCfgs[0]);
@@ -2133,6 +2134,7 @@ static hipError_t launch_tiled_cfg(int cfg, const GemmArgs & a, int nblocks, hip
         case 32: return launch_1w<128, 96, 2, 2, 9>(a, nblocks, st);
         case 33: return launch_1w<128, 64, 2, 2, 9>(a, nblocks, st);
         case 34: return launch_1w<64, 128, 2, 2, 9>(a, nblocks, st);
+        case 35: return launch_1w<256, 256, 2, 2, 5>(a, nblocks, st);
         default: return hipErrorInvalidValue;
     }
 }

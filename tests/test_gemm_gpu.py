@@ -593,7 +593,7 @@ def test_pack_clear_then_accumulating_gemm(mx):
 # and N off every tile, two members of one panel (the second at a row that is no multiple of 16),
 # and an output whose rows are not 16-byte aligned.
 @pytest.mark.parametrize("K,ksplit", [(96, 1), (1312, 1), (1312, 3), (4096, 8)])
-@pytest.mark.parametrize("cfg", range(25, 35))
+@pytest.mark.parametrize("cfg", range(25, 36))
 def test_one_wave_gemm(mx, monkeypatch, cfg, K, ksplit):
     import torch
     monkeypatch.setenv("MI355X_GEMM_CFG", str(cfg))
