@@ -1090,14 +1090,17 @@ int flash_attn_device(Ctx * c, mi355x_tensor * dst) {
     const mi355x_tensor * v = dst->src[2];
     const mi355x_tensor * m = dst->src[3];
     const size_t qb = nbytes(q), kb = nbytes(k), vb = nbytes(v), mb = m ? nbytes(m) : 0, ob = nbytes(dst);
+    // V as a view of K's first dims (the absorbed MLA): uploaded once, and the kernel sees the view
+    const bool v_in_k = v->data == k->data && v->type == k->type && v->nb[1] == k->nb[1] && v->nb[2] == k->nb[2] &&
+                        vb <= kb;
     TRY(c->fa_q.ensure(qb, c->stream));
     TRY(c->fa_k.ensure(kb, c->stream));
-    TRY(c->fa_v.ensure(vb, c->stream));
+    if (!v_in_k) TRY(c->fa_v.ensure(vb, c->stream));
     if (m) TRY(c->fa_m.ensure(mb, c->stream));
     TRY(c->fa_o.ensure(ob, c->stream));
     TRY(upload(c, c->fa_q.p, q->data, qb));
     TRY(upload(c, c->fa_k.p, k->data, kb));
-    TRY(upload(c, c->fa_v.p, v->data, vb));
+    if (!v_in_k) TRY(upload(c, c->fa_v.p, v->data, vb));
     if (m) TRY(upload(c, c->fa_m.p, m->data, mb));
     mi355x_fa_args a;
     memset(&a, 0, sizeof a);
@@ -1107,7 +1110,7 @@ int flash_attn_device(Ctx * c, mi355x_tensor * dst) {
     a.k_dev = (const uint16_t *)c->fa_k.p;
     a.k_nb1 = (int64_t)(k->nb[1] / 2);
     a.k_nb2 = (int64_t)(k->nb[2] / 2);
-    a.v_dev = (const uint16_t *)c->fa_v.p;
+    a.v_dev = (const uint16_t *)(v_in_k ? c->fa_k.p : c->fa_v.p);
     a.v_nb1 = (int64_t)(v->nb[1] / 2);
     a.v_nb2 = (int64_t)(v->nb[2] / 2);
     a.mask_dev = m ? (const uint16_t *)c->fa_m.p : nullptr;

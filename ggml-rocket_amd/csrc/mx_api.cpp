@@ -382,6 +382,17 @@ static bool fa_is_wide(const mi355x_fa_args * a) {
 }
 static constexpr int64_t FA_WIDE_MAX_KV = 1 << 20;
 
+// The absorbed MLA (dk 576, dv 512) whose V is the first 512 dims of K, the same pointer and strides:
+// the fused kernel (mx_fa_mla.hip), which reads one cache for both products and addresses a KV head's
+// keys by 32-bit byte offsets. It wins from one token on (16 heads, n_kv 4096, two GEMMs against fused:
+// T 1 60 / 41 us, T 512 247 / 116; T 16 n_kv 1024 43 / 34), so everything else about the call is free.
+// Other head dims past 256, V elsewhere and n_kv past its class table take the two-GEMM path.
+static bool fa_is_mla(const mi355x_fa_args * a) {
+    return a->D == 576 && a->DV == 512 && a->v_dev == a->k_dev && a->v_nb1 == a->k_nb1 &&
+           (a->HK == 1 || a->v_nb2 == a->k_nb2) && a->k_nb1 >= a->D && a->KV >= 1 && a->KV <= mx::FA_MLA_MAX_KV &&
+           ((int64_t)a->KV + 64) * a->k_nb1 * 2 < 0x7FFFFFFF && (int64_t)a->H * a->T < ((int64_t)1 << 30);
+}
+
 static int fa_check(const mi355x_fa_args * a) {
     if (!a || !a->q_dev || !a->k_dev || !a->v_dev || !a->dst_dev) return MI355X_E_ARG;
     const bool wide = fa_is_wide(a);
@@ -504,6 +515,28 @@ static FaPlan fa_plan(const mi355x_fa_args * a, int nsplit_req) {
     return best;
 }
 
+// The fused MLA's launch arguments. KV split: a block takes about 2.9 us a key tile after some 12 us
+// of prologue (measured at 16 heads, 512 queries, n_kv 4096); a split writes its partial rows and
+// reads them back in the combine launch.
+static mx::FaArgs fa_mla_lower(const mi355x_fa_args * a) {
+    mx::FaArgs f = fa_lower(a, 1);
+    f.D = 576;
+    f.DV = 512;
+    const int ntiles = f.kvp / 64, cus = device_cus();
+    const int64_t nb = mx::fa_mla_blocks(f);
+    const double part_mb = (double)a->T * a->H * 512 * 8.0 / 1e6;
+    double best = 0.0;
+    for (int ns = 1; ns <= std::min(std::max(ntiles / 4, 1), 64); ns++) {
+        const int64_t rounds = (nb * ns + cus - 1) / cus;
+        const double us = (double)rounds * (12.0 + ((ntiles + ns - 1) / ns) * 2.9) + (ns > 1 ? 3.0 + ns * part_mb / 6.0 : 0.0);
+        if (ns == 1 || us < best - 1e-9) {
+            best = us;
+            f.nsplit = ns;
+        }
+    }
+    return f;
+}
+
 MI355X_API int mi355x_flash_attn_auto_split(const mi355x_fa_args * a) {
     if (fa_check(a) != MI355X_OK || fa_is_wide(a)) return 1;
     return fa_plan(a, 0).nsplit;
@@ -511,7 +544,8 @@ MI355X_API int mi355x_flash_attn_auto_split(const mi355x_fa_args * a) {
 
 MI355X_API size_t mi355x_flash_attn_workspace(const mi355x_fa_args * a, int nsplit) {
     if (fa_check(a) != MI355X_OK) return 0;
-    if (fa_is_wide(a)) return fa_wide_layout(a).total;   // no KV split on this path
+    if (fa_is_mla(a)) return fa_layout(fa_mla_lower(a)).total;   // its own KV split
+    if (fa_is_wide(a)) return fa_wide_layout(a).total;           // no KV split on this path
     if (nsplit <= 0) nsplit = fa_plan(a, 0).nsplit;
     if (nsplit > 64) return 0;
     return fa_layout(fa_lower(a, nsplit)).total;
@@ -528,6 +562,17 @@ MI355X_API int mi355x_flash_attn_ex(const mi355x_fa_args * a, int nsplit, int fl
     const int st = fa_check(a);
     if (st != MI355X_OK) return st;
     if (a->T == 0) return MI355X_OK;
+    if (fa_is_mla(a)) {
+        mx::FaArgs f = fa_mla_lower(a);
+        const FaLayout L = fa_layout(f);
+        if (!workspace_dev || workspace_bytes < L.total || !aligned(workspace_dev, 256)) return MI355X_E_NOMEM;
+        char * ws = (char *)workspace_dev;
+        f.cls = (uint8_t *)(ws + L.cls);
+        f.kzero = (uint16_t *)(ws + L.zero);
+        f.part_o = (float *)(ws + L.po);
+        f.part_ml = (float *)(ws + L.pml);
+        return hip_status(mx::launch_fa_mla(f, true, S(stream)));
+    }
     if (fa_is_wide(a)) {
         const FaWideLayout L = fa_wide_layout(a);
         if (!workspace_dev || workspace_bytes < L.total || !aligned(workspace_dev, 256)) return MI355X_E_NOMEM;

@@ -924,6 +924,22 @@ size_t fa_max_kv(int dk, int dv) {
     return (size_t)(FA_LDS_MAX - ring - 64) / 4 / 16 * 16 * FA_BKV;
 }
 
+hipError_t launch_fa_prep(const FaArgs & a, hipStream_t st) {
+    hipLaunchKernelGGL(fa_prep_kernel, dim3(fa_prep_blocks(a)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+template <int DV>
+static hipError_t fa_launch_combine(const FaArgs & a, hipStream_t st) {
+    const int64_t rows = (int64_t)a.T * a.H;
+    const int rpb = 256 / (DV / 4);
+    hipLaunchKernelGGL(fa_combine_kernel<DV>, dim3((unsigned)((rows + rpb - 1) / rpb)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+hipError_t launch_fa_combine(const FaArgs & a, hipStream_t st) {
+    return a.DV == 512 ? fa_launch_combine<512>(a, st) : hipErrorInvalidValue;
+}
+
 template <int DK, int DV, int NT, bool SC>
 static hipError_t fa_launch_main(const FaArgs & a, int nb, hipStream_t st) {
     static bool done = false;
@@ -940,10 +956,7 @@ static hipError_t fa_launch_main(const FaArgs & a, int nb, hipStream_t st) {
 template <int DK, int DV>
 static hipError_t fa_launch_all(const FaArgs & a, int nb, bool prep, hipStream_t st) {
     hipError_t e = hipSuccess;
-    if (prep) {
-        hipLaunchKernelGGL(fa_prep_kernel, dim3(fa_prep_blocks(a)), dim3(256), 0, st, a);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
+    if (prep && (e = launch_fa_prep(a, st)) != hipSuccess) return e;
     if constexpr (DV <= 128) {
         if (a.tasks == 2)
             e = a.softcap != 0.0f ? fa_launch_main<DK, DV, 2, true>(a, nb, st) : fa_launch_main<DK, DV, 2, false>(a, nb, st);
@@ -953,10 +966,7 @@ static hipError_t fa_launch_all(const FaArgs & a, int nb, bool prep, hipStream_t
         e = a.softcap != 0.0f ? fa_launch_main<DK, DV, 4, true>(a, nb, st) : fa_launch_main<DK, DV, 4, false>(a, nb, st);
     }
     if (e != hipSuccess || a.nsplit == 1) return e;
-    const int64_t rows = (int64_t)a.T * a.H;
-    const int rpb = 256 / (DV / 4);
-    hipLaunchKernelGGL(fa_combine_kernel<DV>, dim3((unsigned)((rows + rpb - 1) / rpb)), dim3(256), 0, st, a);
-    return hipGetLastError();
+    return fa_launch_combine<DV>(a, st);
 }
 
 hipError_t launch_fa(const FaArgs & a, bool prep, hipStream_t st) {

@@ -1,7 +1,7 @@
 // SPDX-License-Identifier: MIT
-// FLASH_ATTN_EXT for head dims past the fused kernel's 256: the absorbed MLA of DeepSeek-style
-// models (dk 576, dv 512) and any dk % 32 == 0, dv % 8 == 0 up to 1024, the claim range of
-// ggml-rocket.cpp:7740-7760. Same semantics as the fused kernel (ggml-rocket.cpp:5444-5691):
+// FLASH_ATTN_EXT for head dims past the fused kernel's 256: any dk % 32 == 0, dv % 8 == 0 up to 1024,
+// the claim range of ggml-rocket.cpp:7740-7760; the absorbed MLA (dk 576, dv 512) too where its V is
+// not the first dims of K (mx_fa_mla.hip has that case). Same semantics as the fused kernel (ggml-rocket.cpp:5444-5691):
 //   O[t,h,:] = softmax_j( cap(scale * q[h,t].k[hk,j]) + mask[t,j] ) . v[hk,j,:],  hk = h / (H/HK)
 // computed as two GEMMs around a softmax pass, per KV head and chunk of query rows:
 //   Q16 = fp16(scale * q), row-scaled like the activation pack; its rows are ordered (local

@@ -113,6 +113,13 @@ int fa_prep_blocks(const FaArgs & a);
 bool fa_dims_supported(int dk, int dv);   // fa_pad_dims: dk, dv <= 256, multiples of 8
 size_t fa_max_kv(int dk, int dv);          // the longest KV range one launch takes
 hipError_t launch_fa(const FaArgs & a, bool prep, hipStream_t st);
+hipError_t launch_fa_prep(const FaArgs & a, hipStream_t st);      // the mask classes (every fused kernel)
+hipError_t launch_fa_combine(const FaArgs & a, hipStream_t st);   // merges KV splits at DV 512
+
+// the fused absorbed MLA (dk 576, dv 512, V the first 512 dims of K)
+constexpr int FA_MLA_MAX_KV = 172032;   // its class bytes' room in LDS
+int fa_mla_blocks(const FaArgs & a);   // per KV split
+hipError_t launch_fa_mla(const FaArgs & a, bool prep, hipStream_t st);
 
 // zc (optional): an F32 output [M][ldzc] whose first zn columns the pack also clears
 hipError_t launch_pack_act(const float * X, int64_t ldx, int M, int K, uint16_t * A16, int64_t lda,

@@ -268,7 +268,9 @@ MI355X_API int mi355x_flash_attn_auto_split(const mi355x_fa_args * a);
 /* Workspace bytes for `nsplit` KV splits (0 = auto): the per-tile mask classes, 16 zero bytes
  * (the source of zero-padded head dims) and, for nsplit > 1, the partial outputs and their
  * (max, sum); for head dims past 256, the fp16 queries, one KV head's keys and transposed
- * values, and a chunk of query rows' scores and fp16 P (at most 64 MiB of F32 scores). Always
+ * values, and a chunk of query rows' scores and fp16 P (at most 64 MiB of F32 scores), except for
+ * the absorbed MLA with V inside K (mi355x_flash_attn), whose classes and partials are as above with
+ * a split of its own. Depends on whether v_dev equals k_dev: ask with the call's pointers. Always
  * non-zero for a valid op; the workspace must be 256-byte aligned. */
 MI355X_API size_t mi355x_flash_attn_workspace(const mi355x_fa_args * a, int nsplit);
 
@@ -279,7 +281,8 @@ MI355X_API size_t mi355x_flash_attn_workspace(const mi355x_fa_args * a, int nspl
  * kernels are built for (64, 64), (128, 128), the MLA (192, 128) and (256, 256); other dims run
  * zero-padded on the smallest that holds them); past 256 (the absorbed MLA's 576 / 512: D % 32
  * == 0, DV % 8 == 0, both up to 1024) as two GEMMs around a softmax pass over a bounded chunk
- * of query rows at a time, with no KV split; H % HK == 0; max_bias
+ * of query rows at a time, with no KV split, or, for 576 / 512 with V the first 512 dims of K (v_dev ==
+ * k_dev, the same strides), fused, choosing its own KV split; H % HK == 0; max_bias
  * must be 0 (no ALiBi); the mask
  * covers [T][KV] with mask_nb1 % 4 == 0; q rows and dst rows 16-byte aligned; k/v rows 16-byte
  * aligned. Rows whose every key is masked are written as zeros. Replaces

@@ -319,3 +319,49 @@ def test_fa_classes_ready_reuses_the_mask_classes(mx, nsplit):
         if layer == 0:
             want = O.flash_attn(Q, K16, V16, M16, scale)
             assert np.all(got[17] == 0.0) and float(np.abs(got - want).max()) <= 2e-2
+
+
+@pytest.mark.parametrize("T,H,HK,KV,softcap,mask", [(70, 16, 1, 389, 0.0, "holes"), (70, 16, 1, 389, 30.0, "holes"),
+                                                    (1, 16, 1, 1500, 0.0, None), (3, 1, 1, 1, 0.0, None),
+                                                    (37, 10, 2, 1000, 0.0, "causal"), (200, 3, 1, 640, 0.0, "skip")])
+def test_fa_mla_fused(mx, T, H, HK, KV, softcap, mask):
+    """The absorbed MLA with V the first 512 dims of K runs fused (64 query rows a block, 64-key tiles, the
+    key range split across blocks): a mask with holes and a fully masked row, whole key tiles masked
+    in the middle of the range, no mask, heads that do not divide a block's 64 rows, two KV heads, n_kv
+    off the tile and of one key, and the output columns past dv untouched; against the oracle and the
+    two-GEMM path (the same call with V copied elsewhere)."""
+    import torch
+    D, DV = 576, 512
+    Q = O.fill_normal((H, T, D), 3990 + T)
+    K16 = O.f32_to_f16_bits(O.fill_normal((HK, KV, D), 3991 + KV))
+    M16 = m = None
+    if mask:
+        pad = (KV + 7) // 8 * 8
+        M = np.full((T, pad), 7.0, np.float32)
+        M[:, :KV] = causal_mask(T, KV)
+        if mask == "holes":
+            M[:, :KV][O.fill_uniform((T, KV), 3993, 1.0) > 0.8] = -np.inf
+            M[5, :] = -np.inf
+        if mask == "skip":
+            M[:, 128:320] = -np.inf
+        M16 = O.f32_to_f16_bits(M)
+        m = torch.from_numpy(M16.view(np.float16)).cuda()
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(D)))
+    V16 = np.ascontiguousarray(K16[:, :, :DV])
+    want = O.flash_attn(Q, K16, V16, M16, scale, softcap=softcap)
+    q = torch.from_numpy(Q).cuda()
+    k = torch.from_numpy(K16.view(np.float16)).cuda()
+    wide = torch.full((T, H, DV + 16), float("nan"), dtype=torch.float32, device="cuda")
+    mx.flash_attn(q, k, k[..., :DV], m, scale, softcap=softcap, out=wide[:, :, :DV])
+    two = mx.flash_attn(q, k, torch.from_numpy(V16.view(np.float16)).cuda(), m, scale, softcap=softcap)
+    torch.cuda.synchronize()
+    w = wide.cpu().numpy()
+    assert np.isnan(w[:, :, DV:]).all(), "wrote past dv"
+    got = w[:, :, :DV]
+    if mask == "holes":
+        assert np.all(got[5] == 0.0)
+    r = compare(want, got)
+    print(f"fused MLA T={T} H={H}/{HK} KV={KV}: {r}")
+    assert r["nonfinite"] == 0 and r["max_abs"] <= 2e-2 and r["range_err"] <= 1e-2, r
+    # both round Q and P to fp16 (2^-11 relative each) and sum in fp32
+    assert np.abs(got - two.cpu().numpy()).max() <= 4 * 2.0 ** -11 * max(np.abs(want).max(), 1e-6)
