@@ -355,49 +355,58 @@ gemm_kernel(GemmArgs args) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Skinny GEMM (M <= 128): a launch this narrow is bound by how many weight bytes it keeps in
-// flight, not by MFMA rate, so the weight goes from HBM straight into registers and is decoded
-// there into MFMA operands (no LDS round trip for the weight). A block is SK_NW waves over
-// SK_NW*32 weight rows and a run of K groups of CH 64-deep chunks; lane (r, g) of a wave loads
+// Skinny GEMM (M <= 128): a launch this narrow is bound by latency, not by MFMA rate or HBM, so the
+// weight goes from HBM straight into registers and is decoded there into MFMA operands (no LDS round
+// trip for the weight). A block is KW ways along K of NW waves over NW*32 weight rows, and a run of K
+// groups of CH 64-deep chunks that its ways take in turn (way w groups w, w + KW, ..). One way alone
+// leaves one wave a SIMD, whose chain load -> decode -> LDS read -> MFMA nothing hides, and a wave by
+// itself issues VALU at half rate; more blocks instead write more slabs of partials. The ways' sums
+// meet in LDS, added in way order. Lane (r, g) of a wave loads
 // decoder item g of each chunk for weight row r, and the 32 values it decodes (two runs of 16
 // consecutive k) are its B operands for the chunk's four 16-deep MFMA steps, so lane (r, g) of
 // the A operand reads the same k from activation row r. Per group the activation slice
-// [32 MT][64 CH] fp16 sits in LDS (16-byte chunks XOR-swizzled by row), double-buffered, and the
-// weight of the next group is in flight in a second register set while this one is multiplied.
+// [32 MT][64 CH] fp16 sits in LDS (16-byte chunks XOR-swizzled by row), double-buffered per way, and
+// the weight of the next group is in flight in a second register set while this one is multiplied.
 // Issue order matters: one vmcnt counter covers every load in issue order, so each step issues
 // the next group's activation loads before its weight loads (their LDS store then waits for them
 // alone, not for the weight), and nothing consumes a loaded value before the step's compute: the
 // activation's row / K mask is applied at its LDS store, since a select right after a load would
 // make the compiler wait for that load before issuing the next. Past the block's last group the
-// loads re-fetch it and are never multiplied, so the loop body has no branch between a load and
-// its use. The weights are decoded by the packed-fp16 decoders (decode_fast: a quarter to a half
-// of the VALU instructions of the exact decode, which bounded this kernel). Blocks split K: past
-// two ways each writes its slab of the partials, summed in split order by reduce_splits_kernel;
-// two ways add into a zeroed output.
+// loads re-fetch it and are never multiplied (or, where another way still has a group, as zeros), so
+// the loop body has no branch between a load and its use. The weights are decoded by the packed-fp16
+// decoders (decode_fast: a quarter to a half of the VALU instructions of the exact decode). Blocks
+// split K too: past two ways each writes its slab of the partials, summed in split order by
+// reduce_splits_kernel; two ways add into a zeroed output.
+// Whole calls on cold weights, us, one way of four waves -> this: Q4_K 8192 x 3072 M 8 / 64 / 90 / 128
+// 17.0 / 24.1 / 31.5 / 33.3 -> 13.2 / 18.4 / 22.7 / 27.5; 14336 x 4096 M 64 35.2 -> 28.5; Q8_0 3072 x
+// 3072 M 32 17.3 -> 15.5; Q4_K 28672 x 4096 M 64 53.6 -> 41.5. A weight staged by LDS DMA (a kernel
+// that was here for Q6_K and Q8_0) was slower than this everywhere but Q6_K 28672 x 4096 at M 64,
+// where the two are within 1%: Q6_K 8192 x 3072 M 32 24.9 -> 18.4, Q8_0 M 128 32.2 -> 28.1.
 // ---------------------------------------------------------------------------------------------
 constexpr int SK_MAX_M = 128;
-constexpr int SK_NW = 4;
 
-// Two waves per SIMD (two blocks per CU) where the two register sets fit in half the register
-// file without spilling, one otherwise.
-template <int WT, int MT>
-constexpr int skinny_occupancy() {
-    return (WT == T_Q4_K || WT == T_MXFP4 || WT == T_Q4_0 || MT == 1) ? 2 : 1;
+template <int MT, int CH, int NW, int KW>
+constexpr int skinny_lds() {
+    const int ring = KW * 2 * 32 * MT * 8 * CH * 16;
+    const int merge = KW * NW * MT * 16 * WAVE * 4;
+    return ring > merge ? ring : merge;
 }
 
-template <int WT, int MT, int CH>
-__global__ void __launch_bounds__(SK_NW * WAVE)
-__attribute__((amdgpu_waves_per_eu(skinny_occupancy<WT, MT>(), skinny_occupancy<WT, MT>())))
+template <int WT, int MT, int CH, int NW, int KW>
+__global__ void __launch_bounds__(NW * KW * WAVE)
+__attribute__((amdgpu_waves_per_eu(NW * KW / 4, NW * KW / 4)))
 gemm_skinny_kernel(GemmArgs args, int groups_per_block) {
-    constexpr int NW = SK_NW;
     constexpr int CPR = 8 * CH;               // 16-byte chunks per activation row of the slice
     constexpr int ACH = 32 * MT * CPR;        // 16-byte chunks of the slice
     constexpr int APT = ACH / (NW * WAVE);    // per thread
     constexpr int SLICE = ACH * 16;
     static_assert(ACH % (NW * WAVE) == 0, "slice split");
-    __shared__ __align__(16) uint8_t sa[2 * SLICE];
+    extern __shared__ __align__(16) uint8_t sk_smem[];
 
-    const int t = threadIdx.x, lane = t % WAVE, wave = t / WAVE;
+    // t, wave: within this thread's K way, which has its own pair of activation slices
+    const int way = __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * WAVE));
+    const int t = threadIdx.x % (NW * WAVE), lane = t % WAVE, wave = t / WAVE;
+    uint8_t * const sa = sk_smem + way * (2 * SLICE);
     const int lr = lane % 32, lg = lane / 32;
     const int ks = args.ksplit;
     const int split = blockIdx.x % ks;
@@ -435,7 +444,7 @@ gemm_skinny_kernel(GemmArgs args, int groups_per_block) {
         for (int i = 0; i < APT; i++) {
             const int q = t + i * NW * WAVE, r = q / CPR, c = q % CPR;
             const int64_t k = kb + 8 * c;
-            const bool ok = r < args.M && k < args.K;
+            const bool ok = r < args.M && k < args.K && grp <= glast;
             av[i] = *(const u32x4 *)(args.A + (ok ? (int64_t)r * args.lda + k : 0));
             amask |= ok ? (1u << i) : 0u;
         }
@@ -487,31 +496,54 @@ gemm_skinny_kernel(GemmArgs args, int groups_per_block) {
     WLoad<WT> w0[CH], w1[CH];
     u32x4 av[APT];
     uint32_t amask;
-    load_a(av, amask, gb);
-    load_w(w0, gb);
+    // step j multiplies group gb + KW j + way; a way's group past the block's last one is all zeros
+    const int steps = (gn + KW - 1) / KW, g0 = gb + way;
+    load_a(av, amask, g0);
+    load_w(w0, g0);
     store_a(av, amask, 0);
     __syncthreads();
     int q = 0;
-    for (; q + 2 <= gn; q += 2) {
-        load_a(av, amask, gb + q + 1);
-        load_w(w1, gb + q + 1);
+    for (; q + 2 <= steps; q += 2) {
+        load_a(av, amask, g0 + KW * (q + 1));
+        load_w(w1, g0 + KW * (q + 1));
         compute(w0, 0);
         store_a(av, amask, 1);
         __syncthreads();
-        load_a(av, amask, gb + q + 2);
-        load_w(w0, gb + q + 2);
+        load_a(av, amask, g0 + KW * (q + 2));
+        load_w(w0, g0 + KW * (q + 2));
         compute(w1, 1);
         store_a(av, amask, 0);
         __syncthreads();
     }
-    if (q < gn) compute(w0, 0);
+    if (q < steps) compute(w0, 0);
 
     scale_rows(acc, args.scales, 0, lg, args.M);
+    // the ways' sums, added in way order: way w finishes elements [w OWN, (w + 1) OWN) of the tile
+    constexpr int OWN = MT * 16 / KW, WS = NW * MT * 16 * WAVE;
+    float * mg = (float *)sk_smem + wave * (MT * 16 * WAVE) + lane;   // [way][wave][element][lane]
+    __syncthreads();   // the last slices have been read
+#pragma unroll
+    for (int w = 0; w < KW; w++)
+        if (w != way)
+#pragma unroll
+            for (int x = w * OWN; x < (w + 1) * OWN; x++) mg[way * WS + x * WAVE] = acc[x / 16][0][x % 16];
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < KW; w++)
+        if (w == way)
+#pragma unroll
+            for (int x = w * OWN; x < (w + 1) * OWN; x++) {
+                float s = w == 0 ? acc[x / 16][0][x % 16] : mg[x * WAVE];
+#pragma unroll
+                for (int v = 1; v < KW; v++) s += v == w ? acc[x / 16][0][x % 16] : mg[v * WS + x * WAVE];
+                acc[x / 16][0][x % 16] = s;
+            }
     if (!okn || gn == 0) return;
 #pragma unroll
     for (int i = 0; i < MT; i++) {
 #pragma unroll
         for (int e = 0; e < 16; e++) {
+            if ((i * 16 + e) / OWN != way) continue;
             const int r = i * 32 + 8 * (e / 4) + 4 * lg + (e % 4);
             if (r >= args.M) continue;
             float * p = G.C + (int64_t)r * G.ldc + n;
@@ -1455,277 +1487,6 @@ gemm_q4k_kernel(GemmArgs args) {
     }
 }
 
-// ---------------------------------------------------------------------------------------------
-// Skinny GEMM with the weight staged by LDS DMA (M <= 128; Q4_K, Q8_0 and Q6_K weights).
-//
-// The register-staged skinny kernel above keeps one K group of weight in flight per wave beside
-// the one it multiplies, so a block that owns a few groups pays an HBM round trip for nearly each
-// of them. Here the bytes go from HBM into LDS by global_load_lds_dwordx4, which holds them
-// without registers: a ring of NS stages, each one K group (CH 64-deep chunks) of the activation
-// slice and of the weight, NS - 1 groups requested ahead of the one multiplied. A lane's weight
-// item (decoder item g of chunk c of weight row r, as in the register kernel) arrives as NP
-// 16-byte pieces, each DMA'd by the lane that decodes it, to LDS slot
-// ((c * NP + p) * NW + wave) * 1 KB + 16 * lane, so the weight ring is private to its wave; the
-// few bytes of an item that are not 16-byte pieces (a Q8_0 block's scale, a Q6_K block's scales
-// and d) come as the aligned 16 bytes of their plane that hold them, so no register ring (whose
-// loads the compiler would wait for in full at the loop's back edge) is needed. The activation slice is shared by the
-// block's waves and lands XOR-swizzled as in the register kernel: each lane fetches the chunk
-// that belongs at its slot. Per group: wait for this wave's DMA of the group (every group issues
-// the same count, past the block's last group the last one is fetched again, so the count is a
-// constant), one barrier (the slice is complete, and every wave is done with the stage about to
-// be refilled), the DMA of group + NS - 1, then the group's decode and MFMAs.
-// Same decoders, same fp16 products and the same K order per output as the register kernel.
-// ---------------------------------------------------------------------------------------------
-template <int WT> struct SkPieces;
-
-// The aligned 16 bytes of a plane of 2-byte values that hold value `idx` (a plane starts 16-byte
-// aligned and, with N % 16 == 0, spans a whole number of 16-byte chunks, so the chunk is inside
-// it), and the value from that chunk.
-__device__ __forceinline__ const uint8_t * chunk_of16(const uint8_t * plane, int64_t idx) {
-    return plane + ((2 * idx) & ~(int64_t)15);
-}
-// word i (0..3) of c by selects: a runtime index into a vector would go through scratch memory
-__device__ __forceinline__ uint32_t word_of(const u32x4 & c, int i) {
-    const uint32_t lo = (i & 1) ? c[1] : c[0], hi = (i & 1) ? c[3] : c[2];
-    return (i & 2) ? hi : lo;
-}
-__device__ __forceinline__ uint16_t half_in_chunk(const u32x4 & c, int64_t idx) {
-    const int o = (int)((2 * idx) & 15);
-    return (uint16_t)(word_of(c, o >> 2) >> (8 * (o & 3)));
-}
-
-template <> struct SkPieces<T_Q4_K> {   // the block header and this item's 16 bytes of nibbles
-    static constexpr int NP = 2;
-    __device__ static const uint8_t * piece(const uint8_t * W, int64_t rows, int64_t K, int64_t row, int64_t k0,
-                                            int u, int p) {
-        const uint8_t * b = W + (row * (K / 256) + k0 / 256) * 144;
-        return p == 0 ? b : b + 16 + 32 * ((k0 % 256) / 64) + 16 * u;
-    }
-    __device__ static void item(WLoad<T_Q4_K> & w, const u32x4 (&pc)[NP], int64_t, int64_t, int64_t row, int64_t k0,
-                                int, bool ok) {
-        w.hdr = pc[0];
-        w.qs = pc[1];
-        w.j = (int)((k0 % 256) / 64);
-        w.ok = ok;
-    }
-};
-
-template <> struct SkPieces<T_Q8_0> {   // the item's 32 quants and the chunk holding its scale
-    static constexpr int NP = 3;
-    // the item's first value, k0 + 32 u, clamped to 0 past K (the item is then masked)
-    __device__ static int64_t kk(int64_t K, int64_t k0, int u) {
-        const int64_t k = k0 + 32 * u;
-        return k < K ? k : 0;
-    }
-    __device__ static const uint8_t * piece(const uint8_t * W, int64_t rows, int64_t K, int64_t row, int64_t k0,
-                                            int u, int p) {
-        if (p < 2) return W + row * K + kk(K, k0, u) + 16 * p;
-        return chunk_of16(W + rows * K, row * (K / 32) + kk(K, k0, u) / 32);
-    }
-    __device__ static void item(WLoad<T_Q8_0> & w, const u32x4 (&pc)[NP], int64_t rows, int64_t K, int64_t row,
-                                int64_t k0, int u, bool ok) {
-        w.q[0] = pc[0];
-        w.q[1] = pc[1];
-        w.d = half_in_chunk(pc[2], row * (K / 32) + kk(K, k0, u) / 32);
-        w.ok = ok;
-    }
-};
-
-template <> struct SkPieces<T_Q6_K> {   // ql (two runs), qh, the block's 16 scales, the chunk holding d
-    static constexpr int NP = 5;
-    __device__ static const uint8_t * piece(const uint8_t * W, int64_t rows, int64_t K, int64_t row, int64_t k0,
-                                            int u, int p) {
-        const int64_t blk = k0 / 256;
-        const int h = (int)((k0 % 256) / 64) >> 1, l0 = 16 * u;
-        if (p < 2) return W + row * (K / 2) + blk * 128 + 64 * h + l0 + 32 * p;
-        if (p == 2) return W + rows * (K / 2) + row * (K / 4) + blk * 64 + 32 * h + l0;
-        const uint8_t * sc = W + rows * (K / 2) + rows * (K / 4);
-        if (p == 3) return sc + row * (K / 16) + blk * 16;
-        return chunk_of16(sc + rows * (K / 16), row * (K / 256) + blk);
-    }
-    __device__ static void item(WLoad<T_Q6_K> & w, const u32x4 (&pc)[NP], int64_t rows, int64_t K, int64_t row,
-                                int64_t k0, int u, bool ok) {
-        const int64_t blk = k0 / 256;
-        const int q4 = (int)((k0 % 256) / 64), h = q4 >> 1, hi = q4 & 1;
-        w.qla = pc[0];
-        w.qlb = pc[1];
-        w.qh = pc[2];
-        // scales 8h + u + 4hi and that + 2 of the block (sub-blocks (l/16) + {0,2} or + {4,6})
-        const int i0 = 8 * h + u + 4 * hi;
-        const uint32_t s0 = (word_of(pc[3], i0 >> 2) >> (8 * (i0 & 3))) & 0xFFu;
-        const uint32_t s1 = (word_of(pc[3], (i0 + 2) >> 2) >> (8 * ((i0 + 2) & 3))) & 0xFFu;
-        w.sc = s0 | (s1 << 8);
-        w.d = half_in_chunk(pc[4], row * (K / 256) + blk);
-        w.hi = hi;
-        w.ok = ok;
-    }
-};
-
-template <int WT, int MT, int CH, int NS>
-struct SkDmaCfg {
-    static constexpr int NW = SK_NW, THREADS = NW * WAVE;
-    static constexpr int NP = SkPieces<WT>::NP;
-    static constexpr int CPR = 8 * CH;                    // 16-byte chunks per activation row of the slice
-    static constexpr int A_BYTES = 32 * MT * CPR * 16;    // the slice [32 MT][64 CH] fp16
-    static constexpr int PA = A_BYTES / (THREADS * 16);   // activation DMA per wave per group
-    static constexpr int W_BYTES = CH * NP * NW * 1024;   // every wave's pieces of the group
-    static constexpr int STAGE = A_BYTES + W_BYTES;
-    static constexpr int LDS = NS * STAGE;
-    static constexpr int PER = PA + CH * NP;              // DMA per wave per group
-    static_assert(PA >= 1 && PA * THREADS * 16 == A_BYTES, "slice split");
-    static_assert(NS >= 2 && NS <= 4 && LDS <= 160 * 1024, "LDS");
-};
-
-// One block a CU (its ring takes most of the LDS), so one wave a SIMD: the whole register file is
-// the wave's.
-template <int WT, int MT, int CH, int NS>
-__global__ void __launch_bounds__(SK_NW * WAVE)
-__attribute__((amdgpu_waves_per_eu(1, 1)))
-gemm_skinny_dma_kernel(GemmArgs args, int groups_per_block) {
-    using C = SkDmaCfg<WT, MT, CH, NS>;
-    using P = SkPieces<WT>;
-    constexpr int NW = C::NW, CPR = C::CPR, NP = C::NP;
-    extern __shared__ __align__(16) uint8_t smem[];
-
-    const int t = threadIdx.x, lane = t % WAVE, wave = t / WAVE;
-    const int wave_s = __builtin_amdgcn_readfirstlane(wave);
-    const int lr = lane % 32, lg = lane / 32;
-    const int ks = args.ksplit;
-    const int split = blockIdx.x % ks;
-    const int nt = blockIdx.x / ks;
-    int g = 0;
-#pragma unroll
-    for (int i = 1; i < GEMM_MAX_GROUPS; i++)
-        if (i < args.ng && nt >= args.g[i].ntile_begin) g = i;
-    GemmGroup G;
-    G.W = args.g[0].W; G.rows_total = args.g[0].rows_total; G.row0 = args.g[0].row0; G.N = args.g[0].N;
-    G.C = args.g[0].C; G.ldc = args.g[0].ldc; G.ntile_begin = args.g[0].ntile_begin;
-#pragma unroll
-    for (int i = 1; i < GEMM_MAX_GROUPS; i++)
-        if (i == g) {
-            G.W = args.g[i].W; G.rows_total = args.g[i].rows_total; G.row0 = args.g[i].row0; G.N = args.g[i].N;
-            G.C = args.g[i].C; G.ldc = args.g[i].ldc; G.ntile_begin = args.g[i].ntile_begin;
-        }
-    split_target(args, g, split, G.C, G.ldc);
-    const int n = (nt - G.ntile_begin) * (32 * NW) + 32 * wave + lr;   // this lane's weight row
-    const bool okn = n < G.N;
-    const int64_t row = G.row0 + (okn ? n : G.N - 1);
-    const int K = args.K;
-    const int nchunks = (K + 63) / 64;
-    const int ngroups = (nchunks + CH - 1) / CH;
-    const int gb = split * groups_per_block;
-    const int gn = max(0, min(ngroups, gb + groups_per_block) - gb);
-    const int glast = gb + max(gn, 1) - 1;
-    const uint8_t * W = (const uint8_t *)G.W;
-
-    // activation DMA sources: slot q of the slice holds row q / CPR, logical chunk
-    // (q % CPR) ^ (row & 7); rows past M read the last row and k past K the row's first chunk
-    // (finite values, multiplied by zero weights or never stored)
-    const uint16_t * asrc[C::PA];
-    int acol[C::PA];
-#pragma unroll
-    for (int i = 0; i < C::PA; i++) {
-        const int q = (i * NW + wave) * WAVE + lane;
-        const int r = q / CPR, c = (q % CPR) ^ (r & 7);
-        asrc[i] = args.A + (int64_t)min(r, args.M - 1) * args.lda;
-        acol[i] = 8 * c;
-    }
-    // group grp (clamped to the block's last) into stage st
-    auto issue = [&](int grp, int st) __attribute__((always_inline)) {
-        const int gg = min(grp, glast);
-        uint8_t * base = smem + st * C::STAGE;
-        const int64_t kb = (int64_t)gg * CH * 64;
-#pragma unroll
-        for (int i = 0; i < C::PA; i++) {
-            const int64_t k = kb + acol[i];
-            dma16(asrc[i] + (k < K ? k : 0), base + (i * NW + wave_s) * 1024);
-        }
-#pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const int cc = min(gg * CH + c, nchunks - 1);
-            const int64_t k0 = (int64_t)cc * 64;
-#pragma unroll
-            for (int p = 0; p < NP; p++)
-                dma16(P::piece(W, G.rows_total, K, row, k0, lg, p),
-                      base + C::A_BYTES + ((c * NP + p) * NW + wave_s) * 1024);
-        }
-    };
-
-    float16v acc[MT][1];
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) acc[i][0][e] = 0.0f;
-    auto compute = [&](int grp, int st) __attribute__((always_inline)) {
-        const uint8_t * base = smem + st * C::STAGE;
-#pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const int cc = grp * CH + c;
-            u32x4 pc[NP];
-#pragma unroll
-            for (int p = 0; p < NP; p++)
-                pc[p] = *(const u32x4 *)(base + C::A_BYTES + ((c * NP + p) * NW + wave) * 1024 + 16 * lane);
-            WLoad<WT> w;
-            P::item(w, pc, G.rows_total, K, row, (int64_t)min(cc, nchunks - 1) * 64, lg,
-                    okn && cc < nchunks && (WT != T_Q8_0 || (int64_t)cc * 64 + 32 * lg < K));
-            u32x4 b[4];
-            int run0, run1;
-            w.decode_fast(lg, b, run0, run1);
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int ch = 8 * c + (q < 2 ? run0 + 8 * q : run1 + 8 * (q - 2)) / 8;   // slice chunk
-                const half8 bf = __builtin_bit_cast(half8, b[q]);
-#pragma unroll
-                for (int i = 0; i < MT; i++) {
-                    const int r = 32 * i + lr;
-                    const half8 af = *(const half8 *)(base + (r * CPR + (ch ^ (r & 7))) * 16);
-                    acc[i][0] = mfma32(af, bf, acc[i][0]);
-                }
-            }
-        }
-    };
-
-    if (gn > 0) {
-#pragma unroll
-        for (int q = 0; q < NS - 1; q++) issue(gb + q, q);
-        // step j: group gb + j from stage j % NS; the DMA of group gb + j + NS - 1 into the stage
-        // group gb + j - 1 used. Unrolled by NS so the register ring's indices are constants.
-        auto step = [&](int j, auto Sc) __attribute__((always_inline)) {
-            constexpr int S = decltype(Sc)::value;
-            wait_vm_lgkm0<(NS - 2) * C::PER>();
-            __builtin_amdgcn_s_barrier();
-            issue(gb + j + NS - 1, (S + NS - 1) % NS);
-            compute(gb + j, S);
-        };
-        int j = 0;
-        for (; j + NS <= gn; j += NS) {
-            step(j, std::integral_constant<int, 0>());
-            step(j + 1, std::integral_constant<int, 1>());
-            if constexpr (NS > 2) step(j + 2, std::integral_constant<int, 2 % NS>());
-            if constexpr (NS > 3) step(j + 3, std::integral_constant<int, 3 % NS>());
-        }
-        const int left = gn - j;
-        if (left > 0) step(j, std::integral_constant<int, 0>());
-        if (left > 1) step(j + 1, std::integral_constant<int, 1 % NS>());
-        if constexpr (NS > 2) if (left > 2) step(j + 2, std::integral_constant<int, 2 % NS>());
-        wait_vm_lgkm0<0>();   // no DMA may still be writing this block's LDS when it exits
-    }
-
-    scale_rows(acc, args.scales, 0, lg, args.M);
-    if (!okn || gn == 0) return;
-#pragma unroll
-    for (int i = 0; i < MT; i++) {
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const int r = i * 32 + 8 * (e / 4) + 4 * lg + (e % 4);
-            if (r >= args.M) continue;
-            float * p = G.C + (int64_t)r * G.ldc + n;
-            if (ks == 1 || args.part) *p = acc[i][0][e];
-            else unsafeAtomicAdd(p, acc[i][0][e]);
-        }
-    }
-}
-
 // The K-split partials summed in split order, C_g[r][n] = P[0][r][pcol_g + n] + P[1][..] + ...:
 // one thread per 4 columns of a partial row (every group's N and pcol are multiples of 16).
 __global__ void __launch_bounds__(256) reduce_splits_kernel(GemmArgs a, int ks) {
@@ -2351,10 +2112,7 @@ static int choose_cfg(int wt, const GemmArgs & a) {
 __global__ void zero_rows_kernel(GemmArgs args);
 
 // The skinny kernel (configuration 20 for MI355X_GEMM_CFG): every weight format but the tiled
-// fp16 one, M <= SK_MAX_M. Chunk depth CH by M tiles (LDS 32 KB per block, double-buffered). The
-// K split aims at ~240 blocks, about one per CU: fewer leave weight bytes unrequested, more add
-// atomic traffic (the fastest splits measured for Q4_K / Q8_0 at M 32-128, N 3072-14336,
-// K 3072-14336 launch 144-256 blocks).
+// fp16 one, M <= SK_MAX_M.
 constexpr int SKINNY_CFG = 20;
 static_assert(kCfgs[SKINNY_CFG].kind == NONE, "the skinny kernel's id");
 
@@ -2369,97 +2127,85 @@ static bool use_skinny(int wt, const GemmArgs & a) {
     return true;
 }
 
-static int skinny_ch(int M) { return M <= 64 ? 4 : 2; }
-
-// The LDS-DMA skinny kernel (Q4_K, Q8_0, Q6_K): chunk depth CH and ring depth NS per weight type
-// and 32-row M tile, the deepest ring of whole groups that fits in LDS (MI355X_SKINNY_DMA=0
-// selects the register-staged kernel, for comparison).
-// Where it is faster (measured at N 3072-8192, K 3072-8192 on MI355X): Q6_K at every M (M 128:
-// 39.4 against 43.2 us at 8192 x 3072) and Q8_0 past 64 rows; Q4_K, and Q8_0 up to 64 rows, keep
-// the register kernel, which is as fast or faster there (Q4_K M 32: 19.1 against 21.8 us), being
-// bound by its decode and address VALU work rather than by the weight bytes in flight.
-// MI355X_SKINNY_DMA=1 forces this kernel for the three types, 0 the register one (tests).
-// The scale chunks it reads stay inside their planes when every panel's row count is a multiple
-// of 16 (the planes then span whole 16-byte chunks); other panels take the register kernel.
-static bool skinny_dma(int wt, const GemmArgs & a) {
-    if (!(wt == T_Q4_K || wt == T_Q8_0 || wt == T_Q6_K)) return false;
-    const char * e = getenv("MI355X_SKINNY_DMA");
-    const int force = (e && *e) ? atoi(e) : -1;
-    if (force == 0) return false;
-    if (force < 0 && !(wt == T_Q6_K || (wt == T_Q8_0 && a.M > 64))) return false;
-    for (int i = 0; i < a.ng; i++)
-        if (a.g[i].rows_total % 16 != 0) return false;
-    return true;
-}
-static int skinny_dma_ch(int wt, int M) {
-    const int mt = (M + 31) / 32;
-    if (wt == T_Q6_K) return mt <= 1 ? 2 : 1;
-    if (wt == T_Q8_0) return mt <= 2 ? 2 : 1;
-    return mt <= 1 ? 4 : 2;
-}
-static int skinny_chunk_depth(int wt, const GemmArgs & a) {
-    return skinny_dma(wt, a) ? skinny_dma_ch(wt, a.M) : skinny_ch(a.M);
-}
-
-template <int WT, int MT, int CH, int NS>
-static hipError_t launch_skinny_dma1(const GemmArgs & a, int nblocks, int gpb, hipStream_t st) {
-    using C = SkDmaCfg<WT, MT, CH, NS>;
-    auto kern = gemm_skinny_dma_kernel<WT, MT, CH, NS>;
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-        if (e != hipSuccess) return e;
-        attr = true;
-    }
-    hipLaunchKernelGGL(kern, dim3(nblocks), dim3(C::THREADS), C::LDS, st, a, gpb);
-    return hipGetLastError();
-}
-
-template <int WT>
-static hipError_t launch_skinny_dma(const GemmArgs & a, int nblocks, int gpb, hipStream_t st) {
-    const int mt = (a.M + 31) / 32;
-    if constexpr (WT == T_Q6_K) {
-        if (mt == 1) return launch_skinny_dma1<WT, 1, 2, 3>(a, nblocks, gpb, st);
-        if (mt == 2) return launch_skinny_dma1<WT, 2, 1, 4>(a, nblocks, gpb, st);
-        return launch_skinny_dma1<WT, 4, 1, 4>(a, nblocks, gpb, st);
-    } else if constexpr (WT == T_Q8_0) {
-        if (mt == 1) return launch_skinny_dma1<WT, 1, 2, 4>(a, nblocks, gpb, st);
-        if (mt == 2) return launch_skinny_dma1<WT, 2, 2, 3>(a, nblocks, gpb, st);
-        return launch_skinny_dma1<WT, 4, 1, 4>(a, nblocks, gpb, st);
-    } else {
-        if (mt == 1) return launch_skinny_dma1<WT, 1, 4, 3>(a, nblocks, gpb, st);
-        if (mt == 2) return launch_skinny_dma1<WT, 2, 2, 4>(a, nblocks, gpb, st);
-        return launch_skinny_dma1<WT, 4, 2, 3>(a, nblocks, gpb, st);
-    }
-}
-
-static int skinny_ntiles(const GemmArgs & a) {
-    int nt = 0;
-    for (int i = 0; i < a.ng; i++) nt += (a.g[i].N + 32 * SK_NW - 1) / (32 * SK_NW);
-    return nt;
-}
-
-// K groups per block (the split count is ceil(groups / that)), at most `cap` splits
-static int skinny_gpb(int wt, const GemmArgs & a, int cap) {
-    const int ch = skinny_chunk_depth(wt, a);
-    const int ngroups = ((a.K + 63) / 64 + ch - 1) / ch;
-    double blocks = 240.0;
+// A skinny launch's block: nw waves of 32 weight rows, kw ways along K, chunk depth ch; gpb groups
+// a block, ks blocks along K (at most `cap`).
+constexpr int SKINNY_BLOCKS = 256;   // one a CU
+struct SkinnyShape { int ch, nw, kw, gpb, ks; };
+static SkinnyShape skinny_split(const GemmArgs & a, int cap, int ch, int nw, int kw, int ntiles) {
+    int blocks = SKINNY_BLOCKS;
     if (const char * e = getenv("MI355X_SKINNY_BLOCKS")) {   // tuning override
         const int v = atoi(e);
         if (v > 0) blocks = v;
     }
-    const double target = blocks / skinny_ntiles(a);
-    const int ks = std::min(std::max(1, (int)std::lround(target)), cap);
-    return (ngroups + ks - 1) / ks;
+    const int nchunks = (a.K + 63) / 64, ngroups = (nchunks + ch - 1) / ch;
+    const int steps = (ngroups + kw - 1) / kw;
+    const int ks = std::min(std::max(1, blocks / ntiles), cap);
+    const int gpb = (steps + ks - 1) / ks * kw;
+    return {ch, nw, kw, gpb, (ngroups + gpb - 1) / gpb};
+}
+static int skinny_ntiles(const GemmArgs & a, int nw) {
+    int nt = 0;
+    for (int i = 0; i < a.ng; i++) nt += (a.g[i].N + 32 * nw - 1) / (32 * nw);
+    return nt;
+}
+// The block by width and M, measured over N 1024-28672, K 1024-14336, M 8-128 and five weight types
+// (us, Q4_K unless named):
+//   64-wide blocks with four K ways while they make one round of the chip, its K split then the
+//     largest whose blocks (one a CU) stay within it: half the slabs of 128-wide blocks with two ways
+//     (8192 x 3072 M 64 18.6 against 22.8), although each reads the activations for fewer columns;
+//     rounding that split up took a second round (14336 x 4096 M 8 15-30% slower).
+//   past 16384 columns 128-wide blocks with two ways, which need no K split and read the activations
+//     half as often (28672 x 4096 M 64 / 128: 41.5 / 56.3 against 51.1 / 76.9; four ways of one chunk
+//     43.7, spilling past 64 rows).
+//   the same 128-wide blocks, split, where one 64-wide block per tile leaves 3/8 of the chip or more idle
+//     and two take a second round, 129-159 tiles (9536 x 6400, 149 tiles, M 2 / 100: Q8_0 31.6 / 44.0
+//     against 35.5 / 50.9, Q4_K 24.4 / 44.3 against 29.0 / 54.5); at 160 the 64-wide ones are as fast
+//     (10240 x 4096 M 2 Q8_0 24.2, 25.7 at 9984 columns this way).
+//   chunk depth 1 past 64 rows (the slices of four ways fill LDS); up to 64 rows depth 2 (14336 x 4096
+//     M 64 28.5 against 32.0), except where its coarser steps leave a block more of K than depth 1
+//     would (3072 x 3072 M 8: 4 against 3 depth-1 steps, 13.9 against 12.9). A block of one depth-2 step
+//     stays: halving it doubles the slabs (1024 x 1024: 8.2 against 10.5).
+static SkinnyShape skinny_shape(const GemmArgs & a, int cap) {
+    const int nt = skinny_ntiles(a, 2);
+    const bool thin = nt > SKINNY_BLOCKS / 2 && nt < SKINNY_BLOCKS * 5 / 8;
+    if (nt > SKINNY_BLOCKS || thin) return skinny_split(a, cap, 2, 4, 2, skinny_ntiles(a, 4));
+    const SkinnyShape s1 = skinny_split(a, cap, 1, 2, 4, nt);
+    if (a.M > 64) return s1;
+    const SkinnyShape s2 = skinny_split(a, cap, 2, 2, 4, nt);
+    return s2.gpb > s2.kw && s1.gpb < 2 * s2.gpb ? s1 : s2;
+}
+
+template <int WT, int MT, int CH, int NW, int KW>
+static hipError_t launch_skinny1(const GemmArgs & a, int nblocks, int gpb, hipStream_t st) {
+    auto kern = gemm_skinny_kernel<WT, MT, CH, NW, KW>;
+    constexpr int lds = skinny_lds<MT, CH, NW, KW>();
+    static bool attr = false;
+    if (!attr) {
+        const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    hipLaunchKernelGGL(kern, dim3(nblocks), dim3(NW * KW * WAVE), lds, st, a, gpb);
+    return hipGetLastError();
 }
 
 template <int WT>
-static hipError_t launch_skinny(const GemmArgs & a, int nblocks, int gpb, hipStream_t st) {
-    const int mt = (a.M + 31) / 32;
-    if (mt == 1) hipLaunchKernelGGL((gemm_skinny_kernel<WT, 1, 4>), dim3(nblocks), dim3(SK_NW * WAVE), 0, st, a, gpb);
-    else if (mt == 2) hipLaunchKernelGGL((gemm_skinny_kernel<WT, 2, 4>), dim3(nblocks), dim3(SK_NW * WAVE), 0, st, a, gpb);
-    else hipLaunchKernelGGL((gemm_skinny_kernel<WT, 4, 2>), dim3(nblocks), dim3(SK_NW * WAVE), 0, st, a, gpb);
-    return hipGetLastError();
+static hipError_t launch_skinny(const GemmArgs & a, int nblocks, const SkinnyShape & s, hipStream_t st) {
+    auto go = [&](auto m) {
+        constexpr int MT = decltype(m)::value;
+        if (s.nw == 2) {
+            if constexpr (MT <= 2)
+                if (s.ch == 2) return launch_skinny1<WT, MT, 2, 2, 4>(a, nblocks, s.gpb, st);
+            return launch_skinny1<WT, MT, 1, 2, 4>(a, nblocks, s.gpb, st);
+        }
+        return launch_skinny1<WT, MT, 2, 4, 2>(a, nblocks, s.gpb, st);
+    };
+    switch ((a.M + 31) / 32) {
+        case 1: return go(std::integral_constant<int, 1>());
+        case 2: return go(std::integral_constant<int, 2>());
+        case 3: return go(std::integral_constant<int, 3>());
+        default: return go(std::integral_constant<int, 4>());
+    }
 }
 
 // A launch's configuration and K split. A split past two ways takes a slab of the caller's
@@ -2468,7 +2214,7 @@ struct GemmPlan {
     bool skinny;
     int cfg;      // kCfgs index (unused for the skinny kernel)
     int ks;       // K split
-    int gpb;      // skinny kernel: K groups per block
+    SkinnyShape sk;   // skinny kernel: its block and K groups per block
     bool slabs;   // each split writes its slab of the partials (else two ways, added into the output)
 };
 
@@ -2504,10 +2250,8 @@ static GemmPlan plan_gemm(int wt, const GemmArgs & a, int slabs) {
     if (use_skinny(wt, a)) {
         p.skinny = true;
         p.cfg = SKINNY_CFG;
-        p.gpb = skinny_gpb(wt, a, cap);
-        const int ch = skinny_chunk_depth(wt, a);
-        const int ngroups = ((a.K + 63) / 64 + ch - 1) / ch;
-        p.ks = (ngroups + p.gpb - 1) / p.gpb;
+        p.sk = skinny_shape(a, cap);
+        p.ks = p.sk.ks;
         p.slabs = p.ks > 2;
         return p;
     }
@@ -2533,7 +2277,7 @@ hipError_t launch_gemm(int wt, const GemmArgs & a_in, int /*unused*/, hipStream_
                        size_t part_bytes) {
     GemmArgs a = a_in;
     const GemmPlan p = plan_gemm(wt, a, part ? split_slabs(a, part_bytes) : 0);
-    const int bn = p.skinny ? 32 * SK_NW : kCfgs[p.cfg].bn;
+    const int bn = p.skinny ? 32 * p.sk.nw : kCfgs[p.cfg].bn;
     int nt = 0;
     int64_t pcol = 0;
     for (int i = 0; i < a.ng; i++) {
@@ -2556,16 +2300,13 @@ hipError_t launch_gemm(int wt, const GemmArgs & a_in, int /*unused*/, hipStream_
     hipError_t e = hipErrorInvalidValue;
     if (p.skinny) {
         switch (wt) {
-            case T_F16: e = launch_skinny<T_F16>(a, nblocks, p.gpb, st); break;
-            case T_Q8_0: e = skinny_dma(wt, a) ? launch_skinny_dma<T_Q8_0>(a, nblocks, p.gpb, st)
-                                            : launch_skinny<T_Q8_0>(a, nblocks, p.gpb, st); break;
-            case T_Q4_0: e = launch_skinny<T_Q4_0>(a, nblocks, p.gpb, st); break;
-            case T_Q4_K: e = skinny_dma(wt, a) ? launch_skinny_dma<T_Q4_K>(a, nblocks, p.gpb, st)
-                                            : launch_skinny<T_Q4_K>(a, nblocks, p.gpb, st); break;
-            case T_Q5_K: e = launch_skinny<T_Q5_K>(a, nblocks, p.gpb, st); break;
-            case T_Q6_K: e = skinny_dma(wt, a) ? launch_skinny_dma<T_Q6_K>(a, nblocks, p.gpb, st)
-                                            : launch_skinny<T_Q6_K>(a, nblocks, p.gpb, st); break;
-            case T_MXFP4: e = launch_skinny<T_MXFP4>(a, nblocks, p.gpb, st); break;
+            case T_F16: e = launch_skinny<T_F16>(a, nblocks, p.sk, st); break;
+            case T_Q8_0: e = launch_skinny<T_Q8_0>(a, nblocks, p.sk, st); break;
+            case T_Q4_0: e = launch_skinny<T_Q4_0>(a, nblocks, p.sk, st); break;
+            case T_Q4_K: e = launch_skinny<T_Q4_K>(a, nblocks, p.sk, st); break;
+            case T_Q5_K: e = launch_skinny<T_Q5_K>(a, nblocks, p.sk, st); break;
+            case T_Q6_K: e = launch_skinny<T_Q6_K>(a, nblocks, p.sk, st); break;
+            case T_MXFP4: e = launch_skinny<T_MXFP4>(a, nblocks, p.sk, st); break;
             default: break;
         }
     } else {

@@ -533,7 +533,8 @@ template <> struct WLoad<T_MXFP4X> : WLoad<T_MXFP4> {
 
 template <> struct WLoad<T_Q6_K> {
     u32x4 qla, qlb, qh;   // ql[l], ql[l+32], qh[l] for the thread's 16 l
-    uint32_t sc;          // the 4 int8 scales it needs, packed
+    uint32_t sc;          // the 4 int8 scales of its half's two 64-value runs as loaded: bytes u and u + 2 are its own.
+                          // Picked out in decode: combined here, a pipelined loop waits for them at its back edge
     uint16_t d;
     int hi;               // 0: weights l, l+32 of the half; 1: l+64, l+96
     bool ok;
@@ -547,23 +548,24 @@ template <> struct WLoad<T_Q6_K> {
         const int l0 = 16 * u;
         const uint8_t * ql = W + row * (K / 2) + blk * 128 + 64 * h + l0;
         const uint8_t * qhp = W + rows * (K / 2) + row * (K / 4) + blk * 64 + 32 * h + l0;
-        const int8_t * scp = (const int8_t *)(W + rows * (K / 2) + rows * (K / 4)) + row * (K / 16) + blk * 16 + 8 * h;
+        const uint8_t * scp = W + rows * (K / 2) + rows * (K / 4) + row * (K / 16) + blk * 16 + 8 * h;
         const uint16_t * dp = (const uint16_t *)(W + rows * (K / 2) + rows * (K / 4) + rows * (K / 16)) + row * (K / 256) + blk;
         qla = *(const u32x4 *)ql;
         qlb = *(const u32x4 *)(ql + 32);
         qh = *(const u32x4 *)qhp;
         // scales for sub-blocks (l/16) + {0,2} (hi=0) or + {4,6} (hi=1), l/16 = u
-        const int i0 = u + 4 * hi;
-        sc = (uint32_t)(uint8_t)scp[i0] | ((uint32_t)(uint8_t)scp[i0 + 2] << 8);
+        sc = *(const uint32_t *)(scp + 4 * hi);
         d = *dp;
     }
+    __device__ __forceinline__ float scale0(int u) const { return (float)(int8_t)((sc >> (8 * u)) & 0xFFu); }
+    __device__ __forceinline__ float scale1(int u) const { return (float)(int8_t)((sc >> (8 * u + 16)) & 0xFFu); }
     // packed: the 6-bit codes assembled four bytes at a time (nibble of ql, two bits of qh),
     // each placed under 1024 (magic_pair), less 1024 + 32, times the sub-block scale d * sc
     // rounded to fp16 (zero where the item is masked)
     __device__ __forceinline__ void decode_fast(int u, u32x4 out[4], int & run0, int & run1) const {
         const float df = h2f_bits(d);
-        const half2v DA = splat_h(ok ? df * (float)(int8_t)(sc & 0xFFu) : 0.0f);
-        const half2v DB = splat_h(ok ? df * (float)(int8_t)((sc >> 8) & 0xFFu) : 0.0f);
+        const half2v DA = splat_h(ok ? df * scale0(u) : 0.0f);
+        const half2v DB = splat_h(ok ? df * scale1(u) : 0.0f);
         const half2v OFF = {(_Float16)-1056.0f, (_Float16)-1056.0f};
         const int sn = 4 * hi;
         uint32_t a[8], b[8];
@@ -590,8 +592,8 @@ template <> struct WLoad<T_Q6_K> {
         // four times the VALU work, which bounded the decode pass (28672 x 4096: 84 us of which HBM
         // is 64).
         const float df = h2f_bits(d);
-        const float da = df * (float)(int8_t)(sc & 0xFFu), ca = -32.0f * da;
-        const float db = df * (float)(int8_t)((sc >> 8) & 0xFFu), cb = -32.0f * db;
+        const float da = df * scale0(u), ca = -32.0f * da;
+        const float db = df * scale1(u), cb = -32.0f * db;
         const int sn = 4 * hi;
         uint32_t a[8], b[8];
 #pragma unroll
@@ -637,14 +639,13 @@ template <> struct WLoad<T_Q6_KX> : WLoad<T_Q6_K> {
     struct Lane {
         const uint8_t * ql, * qh, * sc, * d;   // the expert's first group-block in each plane
         uint32_t oql, oqh, osc, od;
-        uint32_t sel;   // byte permute taking scale bytes u and u + 2 of a scale word
     };
     __device__ __forceinline__ static Lane lane(const uint8_t * W, int64_t rows, int64_t K, int64_t row0, int nloc,
                                                 int u) {
         const Q6kxPlanes p = q6kx_planes(rows, K, row0, 0);
         const uint32_t gb = (uint32_t)(nloc / 32) * (uint32_t)(K / 256), r = (uint32_t)(nloc % 32);
         return {W + p.ql, W + p.qh, W + p.sc, W + p.d, gb * 4096 + (32u * u + r) * 16, gb * 2048 + (32u * u + r) * 16,
-                gb * 512 + r * 16, gb * 64 + 2 * r, 0x0C0C0000u | ((uint32_t)(u + 2) << 8) | (uint32_t)u};
+                gb * 512 + r * 16, gb * 64 + 2 * r};
     }
     __device__ __forceinline__ void load(const Lane & L, int64_t K, int64_t k0, bool ok_row) {
         const int64_t blk = k0 / 256;
@@ -656,9 +657,7 @@ template <> struct WLoad<T_Q6_KX> : WLoad<T_Q6_K> {
         qla = *(const u32x4 *)(pl + L.oql);
         qlb = *(const u32x4 *)((pl + 1024) + L.oql);
         qh = *(const u32x4 *)((L.qh + blk * 2048 + h * 1024) + L.oqh);
-        // scales u + 4 hi and u + 4 hi + 2 of the half h: bytes u and u + 2 of one word
-        const uint32_t sw = *(const uint32_t *)((L.sc + blk * 512 + 8 * h + 4 * hi) + L.osc);
-        sc = __builtin_amdgcn_perm(0u, sw, L.sel);
+        sc = *(const uint32_t *)((L.sc + blk * 512 + 8 * h + 4 * hi) + L.osc);
         d = *(const uint16_t *)((L.d + blk * 64) + L.od);
     }
 };

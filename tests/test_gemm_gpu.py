@@ -426,6 +426,27 @@ def test_skinny_mul_mat(mx, wtype, M):
     _assert_bars(ref, got[:, :N], M, N, f"skinny {O.TYPE_NAMES[wtype]} M={M}")
 
 
+# The skinny kernel's block shapes: 64-wide blocks of four K ways (chunk depth 2 and 1; a last block
+# whose ways have no group), three and four M tiles, and past 16384 columns 128-wide blocks of two
+# ways, with odd step counts and (formats of 32-value blocks) K ending half-way through a chunk.
+@pytest.mark.parametrize("M,N,K", [(8, 144, 1280), (70, 144, 1280), (33, 3088, 2816), (20, 16400, 768), (100, 16400, 768)])
+@pytest.mark.parametrize("wtype", SKINNY_TYPES)
+def test_skinny_block_shapes(mx, wtype, M, N, K):
+    import torch
+    K += 0 if wtype in SUPER_BLOCK else 32
+    W = O.fill_normal((N, K), 970 + wtype, 0.0, 0.02)
+    Xf = O.fill_normal((M, K), 971 + M)
+    payload = O.f32_to_f16_bits(W) if wtype == O.F16 else O.quantize(wtype, W)
+    w = mx.upload_weight(wtype, payload, N, K)
+    out = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    mx.mul_mat(wtype, w, N, K, _dev(Xf), out)
+    again = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    mx.mul_mat(wtype, w, N, K, _dev(Xf), again)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    _assert_bars(O.mul_mat(wtype, payload, Xf, N, K), out.cpu().numpy(), M, N, f"skinny shapes {O.TYPE_NAMES[wtype]} M={M}")
+
+
 def test_mxfp4_fast_decode_is_exact(mx, monkeypatch):
     """The skinny kernel's packed MXFP4 decoder gives the exact decode's fp16 values for block
     scales 2^(e-127), e in 80..140 (below 89 every value rounds to zero, to 104 the products are
