@@ -586,14 +586,13 @@ template <> struct WLoad<T_Q6_K> {
         run1 = 32 + 16 * u;
     }
     __device__ __forceinline__ void decode(int u, u32x4 out[4], int & run0, int & run1) const {
-        // d * sc has at most 19 significant bits and 32 times it is exact too, so one fma rounds
-        // (d*sc)*q - 32*(d*sc) exactly as the CPU rounds the product (d*sc)*(q-32). The 6-bit codes
-        // are assembled four bytes at a time, as in the packed form; assembled one by one they cost
-        // four times the VALU work, which bounded the decode pass (28672 x 4096: 84 us of which HBM
-        // is 64).
+        // (d*sc)*(q-32): q - 32 is exact, so the one product rounds as the CPU's does. Not as one fma,
+        // (d*sc)*q - 32*(d*sc): that gives +0 where a negative d*sc meets q = 32 (or q < 32 meets 0), and
+        // a NaN for an infinite d. The 6-bit codes are assembled four bytes at a time, as in the packed
+        // form; assembled one by one they cost four times the VALU work, which bounded the decode pass
+        // (28672 x 4096: 84 us of which HBM is 64).
         const float df = h2f_bits(d);
-        const float da = df * scale0(u), ca = -32.0f * da;
-        const float db = df * scale1(u), cb = -32.0f * db;
+        const float da = mul_rn(df, scale0(u)), db = mul_rn(df, scale1(u));
         const int sn = 4 * hi;
         uint32_t a[8], b[8];
 #pragma unroll
@@ -604,8 +603,8 @@ template <> struct WLoad<T_Q6_K> {
             float fa[4], fb[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                fa[i] = fma_rn(da, (float)((va >> (8 * i)) & 0xFFu), ca);
-                fb[i] = fma_rn(db, (float)((vb >> (8 * i)) & 0xFFu), cb);
+                fa[i] = mul_rn(da, (float)((va >> (8 * i)) & 0xFFu) - 32.0f);
+                fb[i] = mul_rn(db, (float)((vb >> (8 * i)) & 0xFFu) - 32.0f);
             }
             a[2 * w] = pack2h(fa[0], fa[1]);
             a[2 * w + 1] = pack2h(fa[2], fa[3]);

@@ -116,6 +116,31 @@ def test_dequant_f16_bitexact(mx, wtype):
     assert np.array_equal(got, want.reshape(N, K))
 
 
+def test_q6_k_decode_signs_and_infinities(mx):
+    """Q6_K blocks whose (d * scale) is negative, zero of either sign or infinite: every fp16 bit as
+    ggml's (d * sc) * (q - 32), in the row-major and the tiled form. A negative d * scale times a code of
+    32 is -0, an infinite one +-inf except there (NaN, whose bits are free)."""
+    N, K = 48, 512
+    rng = np.random.default_rng(77)
+    blocks = rng.integers(0, 256, size=(N, K // 256, 210), dtype=np.uint8)
+    blocks[:, :, 192:208] = np.array([1, 255, 0, 128, 127, 3, 253, 64] * 2, dtype=np.uint8)   # int8 scales
+    d = np.array([0.02, -0.02, 0.0, -0.0, np.inf, -np.inf, 6e-8, 1000.0], np.float16)
+    blocks[:, :, 208:210] = d[np.arange(N) % 8].view(np.uint8).reshape(N, 1, 2)
+    blocks[:8, :, :192] = 0           # every code 0
+    blocks[8:16, :, :128] = 0         # every code 32: q - 32 is 0
+    blocks[8:16, :, 128:192] = 0xAA
+    want = O.dequantize_f16(O.Q6_K, blocks.reshape(-1), K).reshape(N, K)
+    assert (want == 0x8000).any() and (want == 0).any() and (want == 0x7C00).any() and (want == 0xFC00).any()
+    nan = (want & 0x7FFF) > 0x7C00
+    w = mx.upload_weight(O.Q6_K, blocks.reshape(-1), N, K)
+    for form, got in (("rows", mx.dequant_f16(O.Q6_K, w, N, K).cpu().numpy().view(np.uint16)),
+                      ("tiled", _untile(mx.tile_f16(O.Q6_K, w, N, K).cpu().numpy(), N, K))):
+        got = got.reshape(N, K)
+        assert np.array_equal((got & 0x7FFF) > 0x7C00, nan), form
+        bad = np.argwhere((got != want) & ~nan)
+        assert len(bad) == 0, (form, len(bad), [(int(r), int(c), hex(got[r, c]), hex(want[r, c])) for r, c in bad[:6]])
+
+
 F16_SHAPES = [(64, 32, 8), (384, 256, 256), (3840, 4096, 512), (64, 64, 7), (384, 256, 130),
               (3840, 4096, 250)]
 
