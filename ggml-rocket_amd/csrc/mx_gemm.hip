@@ -2129,15 +2129,17 @@ static bool use_skinny(int wt, const GemmArgs & a) {
 
 // A skinny launch's block: nw waves of 32 weight rows, kw ways along K, chunk depth ch; gpb groups
 // a block, ks blocks along K (at most `cap`).
-constexpr int SKINNY_BLOCKS = 256;   // one a CU
 struct SkinnyShape { int ch, nw, kw, gpb, ks; };
-static SkinnyShape skinny_split(const GemmArgs & a, int cap, int ch, int nw, int kw, int ntiles) {
-    int blocks = SKINNY_BLOCKS;
+// the blocks of one round of the chip: one a CU
+static int skinny_blocks() {
     if (const char * e = getenv("MI355X_SKINNY_BLOCKS")) {   // tuning override
         const int v = atoi(e);
-        if (v > 0) blocks = v;
+        if (v > 0) return v;
     }
-    const int nchunks = (a.K + 63) / 64, ngroups = (nchunks + ch - 1) / ch;
+    return cu_count();
+}
+static SkinnyShape skinny_split(const GemmArgs & a, int cap, int ch, int nw, int kw, int ntiles) {
+    const int blocks = skinny_blocks(), nchunks = (a.K + 63) / 64, ngroups = (nchunks + ch - 1) / ch;
     const int steps = (ngroups + kw - 1) / kw;
     const int ks = std::min(std::max(1, blocks / ntiles), cap);
     const int gpb = (steps + ks - 1) / ks * kw;
@@ -2166,9 +2168,9 @@ static int skinny_ntiles(const GemmArgs & a, int nw) {
 //     would (3072 x 3072 M 8: 4 against 3 depth-1 steps, 13.9 against 12.9). A block of one depth-2 step
 //     stays: halving it doubles the slabs (1024 x 1024: 8.2 against 10.5).
 static SkinnyShape skinny_shape(const GemmArgs & a, int cap) {
-    const int nt = skinny_ntiles(a, 2);
-    const bool thin = nt > SKINNY_BLOCKS / 2 && nt < SKINNY_BLOCKS * 5 / 8;
-    if (nt > SKINNY_BLOCKS || thin) return skinny_split(a, cap, 2, 4, 2, skinny_ntiles(a, 4));
+    const int nt = skinny_ntiles(a, 2), B = skinny_blocks();
+    const bool thin = nt > B / 2 && nt < B * 5 / 8;
+    if (nt > B || thin) return skinny_split(a, cap, 2, 4, 2, skinny_ntiles(a, 4));
     const SkinnyShape s1 = skinny_split(a, cap, 1, 2, 4, nt);
     if (a.M > 64) return s1;
     const SkinnyShape s2 = skinny_split(a, cap, 2, 2, 4, nt);

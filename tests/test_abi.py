@@ -149,6 +149,26 @@ def test_mul_mat_workspace_sizes_the_decode_first_weight():
             assert ws == (poff + part_own if part_own else pack), (wt, M, N, K)
 
 
+def _gemm_slabs(wt, M, N, K):
+    """The K split of a launch that sums slabs (0: one or two ways), from its workspace."""
+    arr = (mx.GemmOut * 1)()
+    arr[0] = mx.GemmOut(0, N, 0, N, 0, N)
+    n = int(mx.lib().mi355x_gemm_workspace(wt, M, K, arr, 1))
+    assert n % (4 * M * N) == 0
+    return n // (4 * M * N)
+
+
+def test_skinny_block_width_follows_the_chip(monkeypatch):
+    """The skinny GEMM's block width and K split are both drawn against one round of the chip (one block a
+    CU; MI355X_SKINNY_BLOCKS stands in for another count here): 64 tiles of 64 columns are 5/8 of 104
+    blocks, so they run as 32 tiles of 128 split three ways, and unsplit where they fill 64 (host-side
+    planning: no GPU needed)."""
+    monkeypatch.setenv("MI355X_SKINNY_BLOCKS", "104")
+    assert _gemm_slabs(mx.Q4_K, 100, 4096, 4096) == 3
+    monkeypatch.setenv("MI355X_SKINNY_BLOCKS", "64")
+    assert _gemm_slabs(mx.Q4_K, 100, 4096, 4096) == 0
+
+
 def test_host_memory_matches_meminfo():
     """The ggml device reports host memory (MemAvailable / MemTotal), as
     ggml_backend_rocket_device_get_memory does (ggml-rocket.cpp:7277-7293), through the host
