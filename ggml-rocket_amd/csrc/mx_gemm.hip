@@ -378,23 +378,25 @@ gemm_kernel(GemmArgs args) {
 // split K too: past two ways each writes its slab of the partials, summed in split order by
 // reduce_splits_kernel; two ways add into a zeroed output.
 // Whole calls on cold weights, us, one way of four waves -> this: Q4_K 8192 x 3072 M 8 / 64 / 90 / 128
-// 17.0 / 24.1 / 31.5 / 33.3 -> 13.2 / 18.4 / 22.7 / 27.5; 14336 x 4096 M 64 35.2 -> 28.5; Q8_0 3072 x
-// 3072 M 32 17.3 -> 15.5; Q4_K 28672 x 4096 M 64 53.6 -> 41.5. A weight staged by LDS DMA (a kernel
-// that was here for Q6_K and Q8_0) was slower than this everywhere but Q6_K 28672 x 4096 at M 64,
-// where the two are within 1%: Q6_K 8192 x 3072 M 32 24.9 -> 18.4, Q8_0 M 128 32.2 -> 28.1.
+// 17.0 / 24.1 / 31.5 / 33.3 -> 13.2 / 18.4 / 22.7 / 27.5; 14336 x 4096 M 64 35.2 -> 28.5; 28672 x 4096 M 64
+// 53.6 -> 41.5; Q8_0 3072 x 3072 M 32 15.5 -> 14.9. A weight staged by LDS DMA (a kernel that was here for
+// Q6_K and Q8_0) was slower: Q6_K 8192 x 3072 M 32 24.9 -> 18.4, Q8_0 M 128 32.2 -> 28.1. One way, two blocks
+// a CU, stays at the widths, depths and types skinny_shape names (up to 32 rows).
 // ---------------------------------------------------------------------------------------------
 constexpr int SK_MAX_M = 128;
 
 template <int MT, int CH, int NW, int KW>
 constexpr int skinny_lds() {
     const int ring = KW * 2 * 32 * MT * 8 * CH * 16;
-    const int merge = KW * NW * MT * 16 * WAVE * 4;
+    const int merge = KW > 1 ? KW * NW * MT * 16 * WAVE * 4 : 0;
     return ring > merge ? ring : merge;
 }
+// waves a SIMD: the block's own, or two blocks' of one K way
+constexpr int skinny_waves(int nw, int kw) { return kw == 1 ? 2 : nw * kw / 4; }
 
 template <int WT, int MT, int CH, int NW, int KW>
 __global__ void __launch_bounds__(NW * KW * WAVE)
-__attribute__((amdgpu_waves_per_eu(NW * KW / 4, NW * KW / 4)))
+__attribute__((amdgpu_waves_per_eu(skinny_waves(NW, KW), skinny_waves(NW, KW))))
 gemm_skinny_kernel(GemmArgs args, int groups_per_block) {
     constexpr int CPR = 8 * CH;               // 16-byte chunks per activation row of the slice
     constexpr int ACH = 32 * MT * CPR;        // 16-byte chunks of the slice
@@ -518,26 +520,29 @@ gemm_skinny_kernel(GemmArgs args, int groups_per_block) {
     if (q < steps) compute(w0, 0);
 
     scale_rows(acc, args.scales, 0, lg, args.M);
-    // the ways' sums, added in way order: way w finishes elements [w OWN, (w + 1) OWN) of the tile
-    constexpr int OWN = MT * 16 / KW, WS = NW * MT * 16 * WAVE;
-    float * mg = (float *)sk_smem + wave * (MT * 16 * WAVE) + lane;   // [way][wave][element][lane]
-    __syncthreads();   // the last slices have been read
+    constexpr int OWN = MT * 16 / KW;   // elements of the tile this way stores
+    if constexpr (KW > 1) {
+        // the ways' sums, added in way order: way w finishes elements [w OWN, (w + 1) OWN) of the tile
+        constexpr int WS = NW * MT * 16 * WAVE;
+        float * mg = (float *)sk_smem + wave * (MT * 16 * WAVE) + lane;   // [way][wave][element][lane]
+        __syncthreads();   // the last slices have been read
 #pragma unroll
-    for (int w = 0; w < KW; w++)
-        if (w != way)
+        for (int w = 0; w < KW; w++)
+            if (w != way)
 #pragma unroll
-            for (int x = w * OWN; x < (w + 1) * OWN; x++) mg[way * WS + x * WAVE] = acc[x / 16][0][x % 16];
-    __syncthreads();
+                for (int x = w * OWN; x < (w + 1) * OWN; x++) mg[way * WS + x * WAVE] = acc[x / 16][0][x % 16];
+        __syncthreads();
 #pragma unroll
-    for (int w = 0; w < KW; w++)
-        if (w == way)
+        for (int w = 0; w < KW; w++)
+            if (w == way)
 #pragma unroll
-            for (int x = w * OWN; x < (w + 1) * OWN; x++) {
-                float s = w == 0 ? acc[x / 16][0][x % 16] : mg[x * WAVE];
+                for (int x = w * OWN; x < (w + 1) * OWN; x++) {
+                    float s = w == 0 ? acc[x / 16][0][x % 16] : mg[x * WAVE];
 #pragma unroll
-                for (int v = 1; v < KW; v++) s += v == w ? acc[x / 16][0][x % 16] : mg[v * WS + x * WAVE];
-                acc[x / 16][0][x % 16] = s;
-            }
+                    for (int v = 1; v < KW; v++) s += v == w ? acc[x / 16][0][x % 16] : mg[v * WS + x * WAVE];
+                    acc[x / 16][0][x % 16] = s;
+                }
+    }
     if (!okn || gn == 0) return;
 #pragma unroll
     for (int i = 0; i < MT; i++) {
@@ -1945,7 +1950,7 @@ static int tiles_of(const GemmArgs & a, int bm, int bn) {
     return nt * ((a.M + bm - 1) / bm);
 }
 
-static int64_t tiles_n_cols(const GemmArgs & a) {
+static int64_t total_cols(const GemmArgs & a) {
     int64_t n = 0;
     for (int i = 0; i < a.ng; i++) n += a.g[i].N;
     return n;
@@ -1957,7 +1962,7 @@ static int64_t tiles_n_cols(const GemmArgs & a) {
 // split, a deeper K more work to share. At least 2 ways, at most 16 and at least 4 K slabs per
 // split. MI355X_GEMM_KSPLIT=<n> forces n (for tuning).
 static double reg_split_est(const GemmArgs & a) {
-    return 6.65 * std::pow((double)a.K, 0.75) / std::sqrt((double)a.M * (double)tiles_n_cols(a));
+    return 6.65 * std::pow((double)a.K, 0.75) / std::sqrt((double)a.M * (double)total_cols(a));
 }
 static int reg_split(const GemmArgs & a, int cap) {
     const int nk = (a.K + BK - 1) / BK;
@@ -2024,7 +2029,7 @@ static double cfg_estimate(const CfgDesc & d, int K, int tiles, double out_mb, i
 // 4096 x 14336 83 us against 91 unsplit). K past ONE_WAVE_MAX_K: the older kernel alone.
 static void choose_tiled(const GemmArgs & a, int slabs, int & cfg, int & ks) {
     const int cus = cu_count();
-    const double out_mb = (double)a.M * (double)tiles_n_cols(a) * 4.0 / 1e6;
+    const double out_mb = (double)a.M * (double)total_cols(a) * 4.0 / 1e6;
     double best = 1e30;
     cfg = 10;
     ks = 1;
@@ -2058,7 +2063,7 @@ static int choose_cfg(int wt, const GemmArgs & a) {
     if (wt == T_F16) {
         int best = -1;
         double best_us = 1e30;
-        const double out_mb = (double)a.M * (double)tiles_n_cols(a) * 4.0 / 1e6;
+        const double out_mb = (double)a.M * (double)total_cols(a) * 4.0 / 1e6;
         for (int c = FIRST_DMA_CFG; c < N_CFGS; c++) {
             if (kCfgs[c].kind != DMA || !cfg_fits(c, wt, a.K)) continue;
             const CfgDesc & d = kCfgs[c];
@@ -2079,7 +2084,7 @@ static int choose_cfg(int wt, const GemmArgs & a) {
     // 1.2-1.4x faster than the register-staged kernel where they apply.
     if (wt == T_Q4_K && a.K % 256 == 0) {
         const int fill = (cus * 7 + 9) / 10;
-        if ((int64_t)a.K >= 2 * tiles_n_cols(a)) return a.M <= 1024 ? 19 : 18;
+        if ((int64_t)a.K >= 2 * total_cols(a)) return a.M <= 1024 ? 19 : 18;
         if (tiles_of(a, 256, 256) >= fill) return 16;
         if (tiles_of(a, 128, 256) >= fill) return 17;
     }
@@ -2089,7 +2094,7 @@ static int choose_cfg(int wt, const GemmArgs & a) {
     // pick is the faster of the two, and 1.1-1.6x faster than the register-staged kernel.
     if (wt == T_Q8_0 && a.K % 256 == 0) {
         const int fill = (cus * 7 + 9) / 10;
-        if (((int64_t)a.K >= 2 * tiles_n_cols(a) && a.M <= 1024) || tiles_of(a, 128, 256) < fill / 2) return 19;
+        if (((int64_t)a.K >= 2 * total_cols(a) && a.M <= 1024) || tiles_of(a, 128, 256) < fill / 2) return 19;
         return 17;
     }
     // a skinny output: split K (see reg_split); otherwise the unsplit tile with the best fill
@@ -2123,13 +2128,18 @@ static bool use_skinny(int wt, const GemmArgs & a) {
     if (wt == T_F16T || a.M > SK_MAX_M) return false;
     if (const char * e = getenv("MI355X_GEMM_CFG"))
         if (*e) return atoi(e) == SKINNY_CFG;
-    if (wt == T_F16 && a.M > 32 && (int64_t)a.K < 2 * tiles_n_cols(a)) return false;
+    if (wt == T_F16 && a.M > 32 && (int64_t)a.K < 2 * total_cols(a)) return false;
     return true;
 }
 
 // A skinny launch's block: nw waves of 32 weight rows, kw ways along K, chunk depth ch; gpb groups
 // a block, ks blocks along K (at most `cap`).
 struct SkinnyShape { int ch, nw, kw, gpb, ks; };
+static int skinny_ntiles(const GemmArgs & a, int nw) {
+    int nt = 0;
+    for (int i = 0; i < a.ng; i++) nt += (a.g[i].N + 32 * nw - 1) / (32 * nw);
+    return nt;
+}
 // the blocks of one round of the chip: one a CU
 static int skinny_blocks() {
     if (const char * e = getenv("MI355X_SKINNY_BLOCKS")) {   // tuning override
@@ -2138,43 +2148,79 @@ static int skinny_blocks() {
     }
     return cu_count();
 }
-static SkinnyShape skinny_split(const GemmArgs & a, int cap, int ch, int nw, int kw, int ntiles) {
-    const int blocks = skinny_blocks(), nchunks = (a.K + 63) / 64, ngroups = (nchunks + ch - 1) / ch;
+static SkinnyShape skinny_split(const GemmArgs & a, int cap, int ch, int nw, int kw, int blocks) {
+    const int nchunks = (a.K + 63) / 64, ngroups = (nchunks + ch - 1) / ch;
     const int steps = (ngroups + kw - 1) / kw;
-    const int ks = std::min(std::max(1, blocks / ntiles), cap);
+    const int ks = std::min(std::max(1, blocks / skinny_ntiles(a, nw)), cap);
     const int gpb = (steps + ks - 1) / ks * kw;
     return {ch, nw, kw, gpb, (ngroups + gpb - 1) / gpb};
 }
-static int skinny_ntiles(const GemmArgs & a, int nw) {
-    int nt = 0;
-    for (int i = 0; i < a.ng; i++) nt += (a.g[i].N + 32 * nw - 1) / (32 * nw);
-    return nt;
-}
-// The block by width and M, measured over N 1024-28672, K 1024-14336, M 8-128 and five weight types
-// (us, Q4_K unless named):
-//   64-wide blocks with four K ways while they make one round of the chip, its K split then the
-//     largest whose blocks (one a CU) stay within it: half the slabs of 128-wide blocks with two ways
-//     (8192 x 3072 M 64 18.6 against 22.8), although each reads the activations for fewer columns;
-//     rounding that split up took a second round (14336 x 4096 M 8 15-30% slower).
-//   past 16384 columns 128-wide blocks with two ways, which need no K split and read the activations
+// The block by width, K, M and type, measured over N 1024-28672, K 1024-14336, M 1-128 and seven weight
+// types (us, Q4_K unless named; B blocks make one round of the chip, one a CU):
+//   64-wide blocks with four K ways while they make one round, the K split then the largest whose
+//     blocks stay within it: half the slabs of 128-wide blocks with two ways (8192 x 3072 M 64 18.6
+//     against 22.8), although each reads the activations for fewer columns; rounding that split up took
+//     a second round (14336 x 4096 M 8 15-30% slower).
+//   past one round 128-wide blocks with two ways, which need no K split and read the activations
 //     half as often (28672 x 4096 M 64 / 128: 41.5 / 56.3 against 51.1 / 76.9; four ways of one chunk
-//     43.7, spilling past 64 rows).
-//   the same 128-wide blocks, split, where one 64-wide block per tile leaves 3/8 of the chip or more idle
-//     and two take a second round, 129-159 tiles (9536 x 6400, 149 tiles, M 2 / 100: Q8_0 31.6 / 44.0
-//     against 35.5 / 50.9, Q4_K 24.4 / 44.3 against 29.0 / 54.5); at 160 the 64-wide ones are as fast
-//     (10240 x 4096 M 2 Q8_0 24.2, 25.7 at 9984 columns this way).
+//     43.7, spilling past 64 rows). Up to 32 rows and from K 4096 on, one way and two blocks a CU where three
+//     K splits of such blocks fit in that, 129-170 tiles (17920 x 4096 M 1: Q8_0 43.5 -> 35.5, Q6_K 55.6 -> 43.5,
+//     MXFP4 32.3 -> 28.5, Q5_K 42.0 -> 34.4), and for Q8_0, unsplit, past that too (28672 x 4096 M 1 / 32 47.6 /
+//     49.1 -> 45.3 / 45.8; other types 0-10% slower).
+//   the same 128-wide blocks of two ways, split three ways, where 64-wide ones make less than 2/3 of a
+//     round and the three splits fit in one, 129-170 tiles of 64 (9536 x 6400, 149 tiles, M 2 / 100: Q8_0 31.6 /
+//     44.0 against 35.5 / 50.9, Q4_K 24.4 / 44.3 against 29.0 / 54.5); from 160 tiles on only past 64 rows, for
+//     Q6_K, Q5_K and F16, or from K 8192 on (10240 x 4096 M 32 20.4 the 64-wide way, 21.9 this; M 100 39.9, 35.0; Q6_K
+//     M 64 37.2, 31.8), and never under K 2560, where the slabs cost more than the idle CUs (9216 x 1792 M 112 MXFP4
+//     28.8 against 21.9).
+//   128-wide blocks too where their K split fills a round better by a sixteenth or more: of one way for
+//     Q8_0 and F16 up to 32 rows, from K 8192 on or where four ways split in three (4608 x 14336 M 1 Q8_0 0.86 of
+//     the time, 4608 x 5376 0.94; the lighter types 0-10% slower there); of two ways past 32 rows, from K 8192 on
+//     (6144 x 8192 M 100 42.0 -> 38.1), and for MXFP4 past 64 rows even where both fill it (4096 x 14336 M 100
+//     41.1 -> 37.9).
 //   chunk depth 1 past 64 rows (the slices of four ways fill LDS); up to 64 rows depth 2 (14336 x 4096
 //     M 64 28.5 against 32.0), except where its coarser steps leave a block more of K than depth 1
 //     would (3072 x 3072 M 8: 4 against 3 depth-1 steps, 13.9 against 12.9). A block of one depth-2 step
-//     stays: halving it doubles the slabs (1024 x 1024: 8.2 against 10.5).
-static SkinnyShape skinny_shape(const GemmArgs & a, int cap) {
-    const int nt = skinny_ntiles(a, 2), B = skinny_blocks();
-    const bool thin = nt > B / 2 && nt < B * 5 / 8;
-    if (nt > B || thin) return skinny_split(a, cap, 2, 4, 2, skinny_ntiles(a, 4));
-    const SkinnyShape s1 = skinny_split(a, cap, 1, 2, 4, nt);
+//     stays while that spares it the slabs (1024 x 1024, two splits: 8.2 against 10.5; but 1536 x 1536 M 16,
+//     three or six: 11.5 against 10.9). In 128-wide blocks depth 1 by the same rule for Q6_K, Q5_K and MXFP4
+//     where they split K (9984 x 4096 M 1 / 64, 22 against 24 chunks: Q6_K 31.2 / 36.2 -> 27.1 / 32.0, MXFP4 M 100
+//     36.0 -> 32.5; Q4_K M 64 0.4 slower), and for Q6_K up to 64 rows where they don't (28672 x 4096 M 64 60.7 ->
+//     59.0).
+//   one way of depth 4, up to 16 rows and K 2048, where its blocks make one step of 4 chunks and the four
+//     ways' one of 8: no merge, and nothing to overlap (2464 x 1792 M 6 11.4 -> 11.0; Q6_K and Q5_K 3% slower).
+static SkinnyShape skinny_shape(int wt, const GemmArgs & a, int cap) {
+    const int B = skinny_blocks(), n2 = skinny_ntiles(a, 2), n4 = skinny_ntiles(a, 4);
+    auto split = [&](int ch, int nw, int kw) { return skinny_split(a, cap, ch, nw, kw, B); };
+    auto chunks = [](const SkinnyShape & s) { return s.gpb * s.ch; };
+    const bool few = a.M <= 32;
+    if (n2 > B) {
+        if (few && a.K >= 4096 && cap >= 3 && 3 * n4 <= 2 * B) return skinny_split(a, cap, 2, 4, 1, 2 * B);
+        if (few && wt == T_Q8_0) return split(2, 4, 1);
+        return split(wt == T_Q6_K && a.M <= 64 ? 1 : 2, 4, 2);
+    }
+    if (2 * n2 > B && 3 * n4 <= B && a.K >= 2560 &&
+        (8 * n2 < 5 * B || (cap >= 3 && (a.M > 64 || wt == T_Q6_K || wt == T_Q5_K || wt == T_F16 || a.K >= 8192)))) {
+        const SkinnyShape s1 = split(1, 4, 2), s2 = split(2, 4, 2);
+        const bool fine = wt == T_Q6_K || wt == T_Q5_K || wt == T_MXFP4;
+        return fine && chunks(s1) < chunks(s2) ? s1 : s2;
+    }
+    const int k2 = B / n2, k4 = B / n4;   // the K splits
+    const bool fuller = 16 * (k4 * n4 - k2 * n2) >= B && cap >= k4;
+    if (few) {
+        if ((wt == T_Q8_0 || wt == T_F16) && fuller && (a.K >= 8192 || (k2 == 3 && a.K >= 1792))) return split(2, 4, 1);
+    } else if (a.K >= 8192 && k2 >= 2) {
+        if (fuller && (a.M > 64 || k2 >= 3)) return split(1, 4, 2);
+        if (wt == T_MXFP4 && a.M > 64 && k2 <= 6 && cap >= k4) return split(1, 4, 2);
+    }
+    const SkinnyShape s1 = split(1, 2, 4);
     if (a.M > 64) return s1;
-    const SkinnyShape s2 = skinny_split(a, cap, 2, 2, 4, nt);
-    return s2.gpb > s2.kw && s1.gpb < 2 * s2.gpb ? s1 : s2;
+    const SkinnyShape s2 = split(2, 2, 4);
+    if (chunks(s1) < chunks(s2) && (s2.gpb > s2.kw || s2.ks > 2)) return s1;
+    if (a.M <= 16 && a.K <= 2048 && s2.gpb == s2.kw && s2.ks > 2 && wt != T_Q6_K && wt != T_Q5_K) {
+        const SkinnyShape s4 = split(4, 4, 1);
+        if (s4.gpb == 1) return s4;
+    }
+    return s2;
 }
 
 template <int WT, int MT, int CH, int NW, int KW>
@@ -2195,11 +2241,15 @@ template <int WT>
 static hipError_t launch_skinny(const GemmArgs & a, int nblocks, const SkinnyShape & s, hipStream_t st) {
     auto go = [&](auto m) {
         constexpr int MT = decltype(m)::value;
+        if constexpr (MT == 1)
+            if (s.kw == 1) return s.ch == 4 ? launch_skinny1<WT, MT, 4, 4, 1>(a, nblocks, s.gpb, st)
+                                            : launch_skinny1<WT, MT, 2, 4, 1>(a, nblocks, s.gpb, st);
         if (s.nw == 2) {
             if constexpr (MT <= 2)
                 if (s.ch == 2) return launch_skinny1<WT, MT, 2, 2, 4>(a, nblocks, s.gpb, st);
             return launch_skinny1<WT, MT, 1, 2, 4>(a, nblocks, s.gpb, st);
         }
+        if (s.ch == 1) return launch_skinny1<WT, MT, 1, 4, 2>(a, nblocks, s.gpb, st);
         return launch_skinny1<WT, MT, 2, 4, 2>(a, nblocks, s.gpb, st);
     };
     switch ((a.M + 31) / 32) {
@@ -2219,12 +2269,6 @@ struct GemmPlan {
     SkinnyShape sk;   // skinny kernel: its block and K groups per block
     bool slabs;   // each split writes its slab of the partials (else two ways, added into the output)
 };
-
-static int64_t total_cols(const GemmArgs & a) {
-    int64_t n = 0;
-    for (int i = 0; i < a.ng; i++) n += a.g[i].N;
-    return n;
-}
 
 // partial slabs [M][sum of N] the workspace holds, at most 64
 static int split_slabs(const GemmArgs & a, size_t part_bytes) {
@@ -2252,7 +2296,7 @@ static GemmPlan plan_gemm(int wt, const GemmArgs & a, int slabs) {
     if (use_skinny(wt, a)) {
         p.skinny = true;
         p.cfg = SKINNY_CFG;
-        p.sk = skinny_shape(a, cap);
+        p.sk = skinny_shape(wt, a, cap);
         p.ks = p.sk.ks;
         p.slabs = p.ks > 2;
         return p;

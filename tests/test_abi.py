@@ -169,6 +169,21 @@ def test_skinny_block_width_follows_the_chip(monkeypatch):
     assert _gemm_slabs(mx.Q4_K, 100, 4096, 4096) == 0
 
 
+def test_skinny_splits_by_shape():
+    """Where the skinny GEMM splits K into slabs on 256 CUs (host-side planning: no GPU needed): three ways in
+    128-wide blocks from 129 to 170 tiles but not at a shallow K, three ways just past one round of 64-wide
+    blocks, and one-step blocks of depth 1 where depth 2 takes slabs too."""
+    for wt, M, N, K, slabs in [(mx.Q6_K, 64, 10240, 4096, 3), (mx.Q4_K, 64, 10240, 4096, 0),
+                               (mx.Q4_K, 100, 10240, 4096, 3), (mx.MXFP4, 112, 9216, 1792, 0),
+                               (mx.MXFP4, 112, 9216, 4096, 3), (mx.Q8_0, 1, 17920, 4096, 3),
+                               (mx.Q8_0, 1, 17920, 2560, 0), (mx.Q8_0, 33, 17920, 4096, 0),
+                               (mx.Q4_K, 16, 1536, 1536, 6), (mx.Q4_K, 16, 1024, 1024, 0),
+                               (mx.Q8_0, 8, 4608, 14336, 7), (mx.Q4_K, 8, 4608, 14336, 3),
+                               (mx.MXFP4, 100, 4096, 14336, 8), (mx.Q4_K, 100, 4096, 14336, 4),
+                               (mx.Q4_K, 8, 2560, 2048, 8), (mx.Q6_K, 8, 2560, 2048, 4)]:
+        assert _gemm_slabs(wt, M, N, K) == slabs, (wt, M, N, K)
+
+
 def test_host_memory_matches_meminfo():
     """The ggml device reports host memory (MemAvailable / MemTotal), as
     ggml_backend_rocket_device_get_memory does (ggml-rocket.cpp:7277-7293), through the host

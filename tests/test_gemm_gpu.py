@@ -472,6 +472,34 @@ def test_skinny_block_shapes(mx, wtype, M, N, K):
     _assert_bars(O.mul_mat(wtype, payload, Xf, N, K), out.cpu().numpy(), M, N, f"skinny shapes {O.TYPE_NAMES[wtype]} M={M}")
 
 
+# The remaining block forms, each at a ragged width and, where the format allows it, with K ending half-way
+# through a chunk: one K way with two blocks a CU (three splits) and unsplit; 128-wide blocks of two ways
+# split three ways, depth 1 and 2; 128-wide blocks that fill a round better, of one way and of two;
+# one way of depth 4 in one step; four ways of depth 1 in one step.
+@pytest.mark.parametrize("wtype,M,N,K", [
+    (O.Q8_0, 20, 16912, 4128), (O.Q6_K, 3, 16912, 4096), (O.Q8_0, 32, 16912, 800),
+    (O.Q6_K, 64, 8464, 2560), (O.MXFP4, 40, 8464, 2592), (O.Q4_K, 100, 10256, 2560), (O.F16, 1, 10256, 2592),
+    (O.Q8_0, 7, 4560, 1824), (O.F16, 32, 4560, 1824), (O.Q5_K, 40, 4560, 8192), (O.Q4_0, 100, 4560, 8224),
+    (O.MXFP4, 128, 4112, 8224), (O.Q4_K, 16, 2464, 1792), (O.MXFP4, 1, 2480, 1824), (O.F16, 9, 2464, 1824),
+    (O.Q8_0, 16, 1552, 1568)])
+def test_skinny_block_forms(mx, wtype, M, N, K):
+    import torch
+    W = O.fill_normal((N, K), 980 + wtype, 0.0, 0.02)
+    Xf = O.fill_normal((M, K), 981 + M)
+    payload = O.f32_to_f16_bits(W) if wtype == O.F16 else O.quantize(wtype, W)
+    w = mx.upload_weight(wtype, payload, N, K)
+    got = []
+    for _ in range(2):
+        wide = torch.full((M, N + 8), float("nan"), dtype=torch.float32, device="cuda")
+        mx.mul_mat(wtype, w, N, K, _dev(Xf), wide[:, :N])
+        torch.cuda.synchronize()
+        got.append(wide.cpu().numpy())
+    assert np.isnan(got[0][:, N:]).all(), "wrote past N"
+    assert np.array_equal(got[0][:, :N], got[1][:, :N]), "launches differ"
+    _assert_bars(O.mul_mat(wtype, payload, Xf, N, K), got[0][:, :N], M, N, f"skinny forms {O.TYPE_NAMES[wtype]} M={M}",
+                 cos_floor=0.999 if M >= 8 else -1.0)
+
+
 def test_mxfp4_fast_decode_is_exact(mx, monkeypatch):
     """The skinny kernel's packed MXFP4 decoder gives the exact decode's fp16 values for block
     scales 2^(e-127), e in 80..140 (below 89 every value rounds to zero, to 104 the products are
