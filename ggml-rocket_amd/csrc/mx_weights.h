@@ -586,25 +586,27 @@ template <> struct WLoad<T_Q6_K> {
         run1 = 32 + 16 * u;
     }
     __device__ __forceinline__ void decode(int u, u32x4 out[4], int & run0, int & run1) const {
-        // (d*sc)*(q-32): q - 32 is exact, so the one product rounds as the CPU's does. Not as one fma,
-        // (d*sc)*q - 32*(d*sc): that gives +0 where a negative d*sc meets q = 32 (or q < 32 meets 0), and
-        // a NaN for an infinite d. The 6-bit codes are assembled four bytes at a time, as in the packed
+        // (d*sc)*(q-32) as (d*sc/4) * (4 (q-32)): both factors are exact, so the one product rounds as the
+        // CPU's does. 4 (q-32) is the signed byte 4q ^ 0x80, which converts in one instruction. Not as one
+        // fma, (d*sc)*q - 32*(d*sc): that gives +0 where a negative d*sc meets q = 32 (or q < 32 meets 0),
+        // and a NaN for an infinite d. The 6-bit codes are assembled four bytes at a time, as in the packed
         // form; assembled one by one they cost four times the VALU work, which bounded the decode pass
         // (28672 x 4096: 84 us of which HBM is 64).
-        const float df = h2f_bits(d);
+        const float df = h2f_bits(d) * 0.25f;
         const float da = mul_rn(df, scale0(u)), db = mul_rn(df, scale1(u));
         const int sn = 4 * hi;
         uint32_t a[8], b[8];
 #pragma unroll
         for (int w = 0; w < 4; w++) {
-            uint32_t va = ((qla[w] >> sn) & 0x0F0F0F0Fu) | (((qh[w] >> sn) & 0x03030303u) << 4);
-            uint32_t vb = ((qlb[w] >> sn) & 0x0F0F0F0Fu) | (((qh[w] >> (sn + 2)) & 0x03030303u) << 4);
-            asm("" : "+v"(va), "+v"(vb));   // each byte converts with one v_cvt_f32_ubyteN
+            auto ror = [](uint32_t x, int n) { return __builtin_amdgcn_alignbit(x, x, (uint32_t)n); };
+            uint32_t va = (ror(qla[w], sn - 2) & 0x3C3C3C3Cu) | ((ror(qh[w], sn - 6) & 0xC0C0C0C0u) ^ 0x80808080u);
+            uint32_t vb = (ror(qlb[w], sn - 2) & 0x3C3C3C3Cu) | ((ror(qh[w], sn - 4) & 0xC0C0C0C0u) ^ 0x80808080u);
+            asm("" : "+v"(va), "+v"(vb));   // each byte converts with one sign-extending v_cvt_f32_i32
             float fa[4], fb[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                fa[i] = mul_rn(da, (float)((va >> (8 * i)) & 0xFFu) - 32.0f);
-                fb[i] = mul_rn(db, (float)((vb >> (8 * i)) & 0xFFu) - 32.0f);
+                fa[i] = mul_rn(da, (float)(int8_t)((va >> (8 * i)) & 0xFFu));
+                fb[i] = mul_rn(db, (float)(int8_t)((vb >> (8 * i)) & 0xFFu));
             }
             a[2 * w] = pack2h(fa[0], fa[1]);
             a[2 * w + 1] = pack2h(fa[2], fa[3]);
