@@ -1721,7 +1721,7 @@ hipError_t launch_pack_act_tiled(const float * X, int64_t ldx, int M, int K, uin
 //        (gemm_f16_cols_kernel), 21 and 22 are that tile with 32-deep stages, three or four of
 //        them in flight where 15 has one of 64 (the 256 x 224 tile's DMA waits are what bounds
 //        it); 23 and 24 are 8 and 14 with eight 32-deep stages. Of these only 8, 9, 10 and 23
-//        also take tiled weights, where 25-34 cannot split K (see choose_cfg).
+//        also take tiled weights, where 25-35 want a K split that has no workspace (choose_tiled).
 //   25-35 one wave per SIMD (gemm_f16_1w_kernel): tiled fp16 weights, any K split.
 //   16-19 Q4_K with every operand by DMA (gemm_q4k_kernel), K % 256 == 0; 18 and 19 split K
 //        (q4k_split). 20 is the skinny kernel's id (use_skinny), not a tile configuration.
@@ -1736,8 +1736,11 @@ hipError_t launch_pack_act_tiled(const float * X, int64_t ldx, int M, int K, uin
 // configuration to measurements on tiled weights, each launch on a weight panel no earlier launch
 // left in the caches: 4-24 at M = 128-2048, N = 1024-28672, K = 2880-14336, mean error 2-9% per
 // configuration, and over 50 shapes the chosen configurations cost 0.6% more than the best
-// measured ones; 25-35 at M = 48-2048, N = 1024-28672, K = 2048-14336 with splits of 1-8, mean error
-// 4-10%, and over 95 shapes the choices cost 1.5% more than the best of all configurations.
+// measured ones; 25-32 at M = 48-2048, N = 1024-28672, K = 2048-14336 with splits of 1-8, mean error
+// 4-10%; 35 has 25's rate with its other two scaled by the tile. 33 and 34, the small tiles, are set to the
+// choices themselves, over 540 random shapes (M 16-2048, N 1024-28672, K 1024-14336, every tile and split):
+// these cost 1.1% more than the best, 37 of them over 5% (fitted like 25-32, both were priced too low: 2.1%,
+// 72 over 5%; 256 x 4096 x 4096 28.5 -> 22.9, 160 x 6144 x 4096 29.3 -> 24.3, 64 x 14336 x 4096 34.6 -> 28.0).
 enum CfgKind { REG = 0, DMA = 1, Q4KDMA = 2, NONE = 3, ONEW = 4 };
 struct CfgDesc {
     int kind;        // REG: gemm_kernel, DMA: gemm_f16_kernel / _cols, Q4KDMA: gemm_q4k_kernel,
@@ -1783,8 +1786,8 @@ static constexpr CfgDesc kCfgs[] = {
     {ONEW, 128, 192, 1, 32, 6.22, 5.35, 13.47, 0.00},  // 30: 64x96, 7 stages
     {ONEW, 128, 128, 1, 32, 5.70, 4.78, 14.32, 0.00},  // 31: 64x64, 9 stages
     {ONEW, 128, 96, 1, 32, 4.66, 3.69, 14.63, 0.00},   // 32: 64x48, 9 stages
-    {ONEW, 128, 64, 1, 32, 4.11, 3.31, 17.89, 0.00},   // 33: 64x32, 9 stages
-    {ONEW, 64, 128, 1, 32, 4.14, 4.19, 15.82, 0.00},   // 34: 32x64, 9 stages
+    {ONEW, 128, 64, 1, 32, 3.32, 1.68, 22.03, 0.00},   // 33: 64x32, 9 stages
+    {ONEW, 64, 128, 1, 32, 3.37, 4.33, 19.99, 0.00},   // 34: 32x64, 9 stages
     {ONEW, 256, 256, 1, 32, 7.98, 10.5, 9.50, 0.00},   // 35: 128x128, 5 stages
 };
 constexpr int FIRST_DMA_CFG = 4;
@@ -2022,28 +2025,42 @@ static double cfg_estimate(const CfgDesc & d, int K, int tiles, double out_mb, i
     return std::sqrt(std::sqrt(p2 * p2 + f2 * f2)) + split;
 }
 
-// Tiled fp16 weights: the one-wave configuration and K split with the least estimate, among the
-// splits whose partials fit (`slabs` of them) and that leave a split at least 512 values of K (16
-// stages; shorter ones are mostly pipeline fill). Without room for two slabs the two-way atomic
-// splits of the older kernel compete too: a deep K over few tiles is still faster split (512 x
-// 4096 x 14336 83 us against 91 unsplit). K past ONE_WAVE_MAX_K: the older kernel alone.
-static void choose_tiled(const GemmArgs & a, int slabs, int & cfg, int & ks) {
+// The least estimate among the tiled-weight configurations of one kind, the one-wave kernel's with every
+// split of at most `slabs` that leaves a split at least 512 values of K (16 stages; shorter ones are
+// mostly pipeline fill), the eight-wave kernel's with their own. Keeps the given best unless beaten.
+static void least_tiled(const GemmArgs & a, int kind, int slabs, double & best, int & cfg, int & ks) {
     const int cus = cu_count();
     const double out_mb = (double)a.M * (double)total_cols(a) * 4.0 / 1e6;
-    double best = 1e30;
-    cfg = 10;
-    ks = 1;
     for (int c = FIRST_DMA_CFG; c < N_CFGS; c++) {
         const CfgDesc & d = kCfgs[c];
-        if (!cfg_fits(c, T_F16T, a.K)) continue;
-        if (d.kind == DMA && slabs >= 2 && a.K <= ONE_WAVE_MAX_K) continue;
+        if (d.kind != kind || !cfg_fits(c, T_F16T, a.K)) continue;
         const int tiles = tiles_of(a, d.bm, d.bn);
         for (int s : {1, 2, 3, 4, 6, 8}) {
-            if (d.kind == DMA ? s != d.ksplit : s > 1 && (s > slabs || a.K / s < 512)) continue;
+            if (kind == DMA ? s != d.ksplit : s > 1 && (s > slabs || a.K / s < 512)) continue;
             const double us = cfg_estimate(d, a.K, tiles, out_mb, s, cus, best);
             if (us < best - 1e-9) { best = us; cfg = c; ks = s; }
         }
     }
+}
+
+// Tiled fp16 weights: the one-wave kernel with its best K split where the workspace holds that split's
+// slabs, whatever room is left beside them: the bytes gemm_split_bytes asks for and any more give the same
+// launch. With fewer, its best split that fits, against the two-way atomic splits of the eight-wave kernel
+// where not even two slabs do (a deep K over few tiles is faster split: 512 x 4096 x 14336 83 us against
+// 91; a launch that wanted no split keeps the one-wave tile: 28 x 2560 x 1536 10.0 us against 11.8). K past
+// ONE_WAVE_MAX_K: the eight-wave kernel alone.
+static void choose_tiled(const GemmArgs & a, int slabs, int & cfg, int & ks) {
+    const bool onew = a.K <= ONE_WAVE_MAX_K;
+    double best = 1e30;
+    cfg = 10;
+    ks = 1;
+    if (onew) {
+        least_tiled(a, ONEW, 64, best, cfg, ks);
+        if (ks <= std::max(slabs, 1)) return;
+        best = 1e30;
+        least_tiled(a, ONEW, slabs, best, cfg, ks);
+    }
+    if (!onew || slabs < 2) least_tiled(a, DMA, slabs, best, cfg, ks);
 }
 
 // Row-major fp16 weights: the DMA configuration with the least estimated time (the CfgDesc model;

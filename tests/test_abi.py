@@ -184,6 +184,24 @@ def test_skinny_splits_by_shape():
         assert _gemm_slabs(wt, M, N, K) == slabs, (wt, M, N, K)
 
 
+def test_tiled_plan_does_not_depend_on_spare_workspace():
+    """A GEMM on tiled weights is planned the same for exactly the workspace it asks for and for any more:
+    where it asks for none (no K split), no workspace must not turn it into the two-way atomic split that a
+    larger buffer would not run (mi355x_gemm_accumulates tells which; host-side planning: no GPU needed)."""
+    L = mx.lib()
+    arr = (mx.GemmOut * 1)()
+    seen = 0
+    for M in (1, 16, 33, 64, 100, 128, 200, 384):
+        for N in (1024, 1536, 2192, 4096, 8192, 14336):
+            for K in (512, 1024, 1536, 1696, 2048, 4096):
+                arr[0] = mx.GemmOut(0, N, 0, N, 0, N)
+                need = int(L.mi355x_gemm_workspace(mx.F16_T, M, K, arr, 1))
+                seen += need == 0
+                for ws in (need, need + 4, need + (1 << 30)):
+                    assert L.mi355x_gemm_accumulates(mx.F16_T, M, K, arr, 1, ws) == 0, (M, N, K, need, ws)
+    assert seen > 50
+
+
 def test_host_memory_matches_meminfo():
     """The ggml device reports host memory (MemAvailable / MemTotal), as
     ggml_backend_rocket_device_get_memory does (ggml-rocket.cpp:7277-7293), through the host
