@@ -56,11 +56,12 @@ __device__ __forceinline__ f32x4 ml_mfma(const half8 & a, const half8 & b, const
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 // The same with b in AGPRs. In assembly, because the compiler copies such an operand to VGPRs for each
-// use. It does not see that this is an MFMA, so the waits it would insert are here: two wait states
-// before each (an operand a vector instruction has just written; under the MFMA before it they cost
-// nothing), and ml_settle between one of these and anything else that touches its accumulator
-// (eight wait states: a 4-pass MFMA's result can be read after seven). Consecutive MFMAs on one
-// accumulator need none.
+// use. It does not see that this is an MFMA, so the waits are here, those it puts around the builtin form
+// on gfx950 (there is no interlock): two wait states between a vector instruction that writes an operand
+// and the MFMA (s_nop 1 before each; under the MFMA before it they cost nothing), eight between the MFMA
+// (16x16x32, 4 passes) and a vector or store instruction that reads its result (s_nop 7: ml_settle, between
+// the last of these and anything else that touches their accumulators), and none between MFMAs that pass
+// one accumulator on.
 __device__ __forceinline__ void ml_mfma_a(const half8 & a, const half8 & b, f32x4 & c) {
     asm volatile("s_nop 1\nv_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(b));
 }
