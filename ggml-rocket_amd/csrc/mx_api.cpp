@@ -387,10 +387,13 @@ static constexpr int64_t FA_WIDE_MAX_KV = 1 << 20;
 // keys by 32-bit byte offsets. It wins from one token on (16 heads, n_kv 4096, two GEMMs against fused:
 // T 1 60 / 41 us, T 512 247 / 116; T 16 n_kv 1024 43 / 34), so everything else about the call is free.
 // Other head dims past 256, V elsewhere and n_kv past its class table take the two-GEMM path.
+static bool fa_mla_sizes(const mi355x_fa_args * a) {
+    return a->D == 576 && a->DV == 512 && a->KV >= 1 && a->KV <= mx::FA_MLA_MAX_KV &&
+           (int64_t)a->H * a->T < ((int64_t)1 << 30);
+}
 static bool fa_is_mla(const mi355x_fa_args * a) {
-    return a->D == 576 && a->DV == 512 && a->v_dev == a->k_dev && a->v_nb1 == a->k_nb1 &&
-           (a->HK == 1 || a->v_nb2 == a->k_nb2) && a->k_nb1 >= a->D && a->KV >= 1 && a->KV <= mx::FA_MLA_MAX_KV &&
-           ((int64_t)a->KV + 64) * a->k_nb1 * 2 < 0x7FFFFFFF && (int64_t)a->H * a->T < ((int64_t)1 << 30);
+    return fa_mla_sizes(a) && a->v_dev == a->k_dev && a->v_nb1 == a->k_nb1 && (a->HK == 1 || a->v_nb2 == a->k_nb2) &&
+           a->k_nb1 >= a->D && ((int64_t)a->KV + 64) * a->k_nb1 * 2 < 0x7FFFFFFF;
 }
 
 static int fa_check(const mi355x_fa_args * a) {
@@ -538,14 +541,17 @@ static mx::FaArgs fa_mla_lower(const mi355x_fa_args * a) {
 }
 
 MI355X_API int mi355x_flash_attn_auto_split(const mi355x_fa_args * a) {
-    if (fa_check(a) != MI355X_OK || fa_is_wide(a)) return 1;
-    return fa_plan(a, 0).nsplit;
+    if (fa_check(a) != MI355X_OK) return 1;
+    if (fa_is_mla(a)) return fa_mla_lower(a).nsplit;
+    return fa_is_wide(a) ? 1 : fa_plan(a, 0).nsplit;
 }
 
 MI355X_API size_t mi355x_flash_attn_workspace(const mi355x_fa_args * a, int nsplit) {
     if (fa_check(a) != MI355X_OK) return 0;
-    if (fa_is_mla(a)) return fa_layout(fa_mla_lower(a)).total;   // its own KV split
-    if (fa_is_wide(a)) return fa_wide_layout(a).total;           // no KV split on this path
+    if (fa_is_wide(a)) {   // by the sizes alone: where V lies decides between the two forms
+        const size_t wide = fa_wide_layout(a).total;
+        return fa_mla_sizes(a) ? std::max(wide, fa_layout(fa_mla_lower(a)).total) : wide;
+    }
     if (nsplit <= 0) nsplit = fa_plan(a, 0).nsplit;
     if (nsplit > 64) return 0;
     return fa_layout(fa_lower(a, nsplit)).total;
@@ -565,13 +571,14 @@ MI355X_API int mi355x_flash_attn_ex(const mi355x_fa_args * a, int nsplit, int fl
     if (fa_is_mla(a)) {
         mx::FaArgs f = fa_mla_lower(a);
         const FaLayout L = fa_layout(f);
-        if (!workspace_dev || workspace_bytes < L.total || !aligned(workspace_dev, 256)) return MI355X_E_NOMEM;
-        char * ws = (char *)workspace_dev;
-        f.cls = (uint8_t *)(ws + L.cls);
-        f.kzero = (uint16_t *)(ws + L.zero);
-        f.part_o = (float *)(ws + L.po);
-        f.part_ml = (float *)(ws + L.pml);
-        return hip_status(mx::launch_fa_mla(f, true, S(stream)));
+        if (workspace_dev && workspace_bytes >= L.total && aligned(workspace_dev, 256)) {
+            char * ws = (char *)workspace_dev;
+            f.cls = (uint8_t *)(ws + L.cls);
+            f.kzero = (uint16_t *)(ws + L.zero);
+            f.part_o = (float *)(ws + L.po);
+            f.part_ml = (float *)(ws + L.pml);
+            return hip_status(mx::launch_fa_mla(f, true, S(stream)));
+        }
     }
     if (fa_is_wide(a)) {
         const FaWideLayout L = fa_wide_layout(a);

@@ -259,7 +259,8 @@ typedef struct mi355x_fa_args {
     float scale, max_bias, softcap;
 } mi355x_fa_args;
 
-/* The KV-split count mi355x_flash_attn uses when called with nsplit = 0. The launch is planned per
+/* The KV-split count mi355x_flash_attn uses when called with nsplit = 0 (for head dims past 256: 1, or the
+ * fused MLA's own, whatever nsplit is). The launch is planned per
  * call: the block layout (two or four 32-query tasks per block) and the split that together
  * minimise an estimate from measured per-step costs; MI355X_FA_TASKS=2|4 in the environment pins
  * the layout (for tests). The result does not depend on the layout beyond fp32 summation order. */
@@ -268,9 +269,9 @@ MI355X_API int mi355x_flash_attn_auto_split(const mi355x_fa_args * a);
 /* Workspace bytes for `nsplit` KV splits (0 = auto): the per-tile mask classes, 16 zero bytes
  * (the source of zero-padded head dims) and, for nsplit > 1, the partial outputs and their
  * (max, sum); for head dims past 256, the fp16 queries, one KV head's keys and transposed
- * values, and a chunk of query rows' scores and fp16 P (at most 64 MiB of F32 scores), except for
- * the absorbed MLA with V inside K (mi355x_flash_attn), whose classes and partials are as above with
- * a split of its own. Depends on whether v_dev equals k_dev: ask with the call's pointers. Always
+ * values, and a chunk of query rows' scores and fp16 P (at most 64 MiB of F32 scores); for the
+ * absorbed MLA's 576 / 512 the larger of that and the fused form's classes and partials (as above, with
+ * a split of its own), so it does not depend on where V lies. Always
  * non-zero for a valid op; the workspace must be 256-byte aligned. */
 MI355X_API size_t mi355x_flash_attn_workspace(const mi355x_fa_args * a, int nsplit);
 

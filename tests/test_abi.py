@@ -202,6 +202,26 @@ def test_tiled_plan_does_not_depend_on_spare_workspace():
     assert seen > 50
 
 
+def test_flash_attn_mla_workspace_and_split():
+    """The absorbed MLA's workspace is sized by the shapes alone: asked for with V inside K (the fused form)
+    it also holds the two-GEMM form of the same call with V elsewhere, and mi355x_flash_attn_auto_split
+    names the fused form's KV split (host-side sizing: no GPU needed)."""
+    L = mx.lib()
+    k, v = 1 << 20, 1 << 24   # never dereferenced on these paths
+
+    def args(vp, T, H, KV, D=576, DV=512):
+        return mx.FaArgs(k, D, T * D, k, D, KV * D, vp, D, KV * D, 0, 0, k, DV, H * DV, D, DV, T, H, KV, 1, 1.0, 0.0, 0.0)
+
+    for T, H, KV in [(1, 16, 4096), (512, 16, 4096), (16, 128, 1024), (3, 1, 1), (1, 16, 200000)]:
+        inside, apart = args(k, T, H, KV), args(v, T, H, KV)
+        need = L.mi355x_flash_attn_workspace(ctypes.byref(inside), 0)
+        assert need == L.mi355x_flash_attn_workspace(ctypes.byref(apart), 0) > 0, (T, H, KV)
+        assert L.mi355x_flash_attn_auto_split(ctypes.byref(apart)) == 1
+    assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 1, 16, 4096))) == 16
+    assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 512, 16, 64))) == 1
+    assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 1, 16, 200000))) == 1   # past its class table
+
+
 def test_host_memory_matches_meminfo():
     """The ggml device reports host memory (MemAvailable / MemTotal), as
     ggml_backend_rocket_device_get_memory does (ggml-rocket.cpp:7277-7293), through the host
