@@ -9,6 +9,8 @@ Plus the prefill attention shapes: 32 query / 8 KV heads, d 128, 512 tokens, n_k
 N(0,1) inputs, causal mask, scale 1/sqrt(128); scored on sampled query rows. Every case runs
 under both block layouts (two or four wave tasks per block).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -365,3 +367,63 @@ def test_fa_mla_fused(mx, T, H, HK, KV, softcap, mask):
     assert r["nonfinite"] == 0 and r["max_abs"] <= 2e-2 and r["range_err"] <= 1e-2, r
     # both round Q and P to fp16 (2^-11 relative each) and sum in fp32
     assert np.abs(got - two.cpu().numpy()).max() <= 4 * 2.0 ** -11 * max(np.abs(want).max(), 1e-6)
+
+
+def _lazy_max_jumps(S, splits):
+    """The finite moves, in log 2, of the fused MLA's running maxima: per (row, split) over 64-key tiles of
+    the scores S [rows][KV], moved only when some row of its 64-row block passes its own by 8."""
+    tiles = [(S[:, j:j + 64].max(1) * np.log2(np.e)) for j in range(0, S.shape[1], 64)]
+    per, jumps = -(-len(tiles) // splits), []
+    for r0 in range(0, S.shape[0], 64):
+        for s in range(splits):
+            run = np.full(min(64, S.shape[0] - r0), -np.inf)
+            for t in tiles[s * per:(s + 1) * per]:
+                new = t[r0:r0 + 64]
+                if (new > run + 8).any():
+                    up = np.maximum(run, new)
+                    fin = np.isfinite(run)
+                    jumps += list((up[fin] - run[fin])[up[fin] > run[fin]])
+                    run = up
+    return np.array(jumps)
+
+
+@pytest.mark.parametrize("T,H,KV,softcap", [(40, 16, 1536, 0.0), (40, 16, 1536, 48.0), (3, 16, 2990, 0.0), (70, 5, 700, 0.0)])
+def test_fa_mla_fused_rescales(mx, T, H, KV, softcap):
+    """Scores that grow along the keys, so every row's running max moves from one finite value to a larger one,
+    by more and by less than the lazy threshold and in different tiles, within and across KV splits, with a
+    fully masked row. Q is whole quarters of its row's max and the scale a power of two, so Q's fp16 form is
+    exact and what is left is P's rounding (2^-11 relative, in the sum over V and in the row sum)."""
+    import torch
+    D, DV, HK = 576, 512, 1
+    Q = np.round(O.fill_uniform((H, T, D), 4990 + T, 4.49)) * 2.0
+    Q[:, :, 7] = 8.0   # the row's max
+    Kf = O.fill_normal((HK, KV, D), 4991 + KV)
+    Kf *= (0.5 + 0.6 * (np.arange(KV) // 64))[None, :, None]
+    K16 = O.f32_to_f16_bits(Kf.astype(np.float32))
+    V16 = np.ascontiguousarray(K16[:, :, :DV])
+    pad = (KV + 7) // 8 * 8
+    M = np.full((T, pad), 7.0, np.float32)
+    M[:, :KV] = causal_mask(T, KV)
+    M[1, :] = -np.inf
+    M16 = O.f32_to_f16_bits(M)
+    scale = 1.0 / 32
+    kd = O.f16_bits_to_f32(K16).astype(np.float64)[0]
+    S = np.einsum("htd,jd->thj", Q.astype(np.float64), kd).reshape(T * H, KV) * scale   # row = token * H + head
+    if softcap:
+        S = softcap * np.tanh(S / softcap)
+    S += np.repeat(M[:, :KV], H, 0)
+    q = torch.from_numpy(Q.astype(np.float32)).cuda()
+    k = torch.from_numpy(K16.view(np.float16)).cuda()
+    m = torch.from_numpy(M16.view(np.float16)).cuda()
+    out = torch.full((T, H, DV), float("nan"), dtype=torch.float32, device="cuda")
+    mx.flash_attn(q, k, k[..., :DV], m, scale, softcap=softcap, out=out)
+    torch.cuda.synchronize()
+    splits = mx.lib().mi355x_flash_attn_auto_split(ctypes.byref(mx._fa_args(q, k, k[..., :DV], m, out, scale, softcap)))
+    jumps = _lazy_max_jumps(S, splits)
+    assert splits > 1 and (jumps > 8).sum() > T * H // 2 and ((jumps > 0.5) & (jumps < 8)).sum() > T, (splits, len(jumps))
+    want = O.flash_attn(Q.astype(np.float32), K16, V16, M16, scale, softcap=softcap)
+    got = out.cpu().numpy()
+    assert np.all(got[1] == 0.0)
+    err, bar = np.abs(got - want).max(), 4 * 2.0 ** -11 * np.abs(O.f16_bits_to_f32(V16)).max()
+    print(f"MLA rescale T={T} KV={KV} softcap={softcap}: {splits} splits, {len(jumps)} moves, err {err:.3g} of {bar:.3g}")
+    assert err <= bar
