@@ -332,27 +332,25 @@ def test_pack_act_tiled_bitexact(mx):
 
 # Every tile configuration of mi355x_gemm, forced through MI355X_GEMM_CFG, on a ragged fused
 # launch (M and both N not multiples of any tile). Configurations 0-3 are the register-staged
-# kernel (every weight layout but the tiled fp16 one); 4-15 and 21-24 the LDS-DMA kernels,
-# which take fp16 weights only, row-major (F16) or tiled (F16_T); 16-19 the kernel with every
-# operand by DMA (K % 256 == 0; Q4_K, and Q8_0 on the 128 x 256 tiles 17 and 19). 20 is the skinny kernel (M <= 128), covered
-# by its own tests.
+# kernel (every weight layout but the tiled fp16 one); 4-15 and 21-24 the eight-wave LDS-DMA kernels,
+# which take row-major fp16 weights (F16), and 8, 9, 10 and 23 tiled ones (F16_T) too; 25-35 the one-wave
+# kernel of tiled weights; 16-19 the kernel with every operand by DMA (K % 256 == 0; Q4_K, and Q8_0 on
+# the 128 x 256 tiles 17 and 19). 20 is the skinny kernel (M <= 128), covered by its own tests. The library
+# ignores a configuration that does not take the weights, so only the pairs that exist are listed.
 REG_CFGS = list(range(0, 4))
 DMA_CFGS = list(range(4, 16)) + [21, 22, 23, 24]
+DMA_TILED = [8, 9, 10, 23]
+ONEW_CFGS = list(range(25, 36))
 QDMA_CFGS = list(range(16, 20))
 F16_T = 0x101
 QUANT = (O.Q4_K, O.MXFP4, O.Q8_0, O.Q6_K, O.Q4_0, O.Q5_K)
+TILE_CONFIGS = ([(O.F16, c) for c in REG_CFGS + DMA_CFGS] + [(F16_T, c) for c in DMA_TILED + ONEW_CFGS] +
+                [(w, c) for w in QUANT for c in REG_CFGS] + [(O.Q4_K, c) for c in QDMA_CFGS] + [(O.Q8_0, c) for c in (17, 19)])
 
 
-@pytest.mark.parametrize("cfg", REG_CFGS + DMA_CFGS + QDMA_CFGS)
-@pytest.mark.parametrize("wtype", [O.F16, O.Q4_K, F16_T, O.MXFP4, O.Q8_0, O.Q6_K, O.Q4_0, O.Q5_K])
+@pytest.mark.parametrize("wtype,cfg", TILE_CONFIGS)
 def test_gemm_every_tile_config(mx, monkeypatch, cfg, wtype):
     import torch
-    if cfg in DMA_CFGS and wtype in QUANT:
-        pytest.skip("the LDS-DMA configurations take fp16 weights only")
-    if cfg in REG_CFGS and wtype == F16_T:
-        pytest.skip("the register-staged configurations do not read the tiled layout")
-    if cfg in QDMA_CFGS and wtype != O.Q4_K and not (wtype == O.Q8_0 and cfg in (17, 19)):
-        pytest.skip("the all-DMA configurations take Q4_K weights, and Q8_0 on the 128-row tiles")
     monkeypatch.setenv("MI355X_GEMM_CFG", str(cfg))
     K, M, Ns = 1280, 300, (528, 144)
     Xf = O.fill_normal((M, K), 900 + cfg)
@@ -533,12 +531,12 @@ def test_mxfp4_fast_decode_is_exact(mx, monkeypatch):
 
 @pytest.mark.parametrize("M", [1, 32, 64, 100, 128])
 @pytest.mark.parametrize("wtype", [O.Q8_0, O.Q4_K, O.Q6_K])
-def test_skinny_dma_matches_register_kernel(mx, monkeypatch, wtype, M):
-    """The skinny kernel with the weight staged by LDS DMA (Q8_0, Q4_K, Q6_K) against the
-    register-staged one (MI355X_SKINNY_DMA=0) on the same packed activations: both walk the same
-    64-deep chunks in the same order with the same decoders, so where their K splits coincide
-    (one split: K within one block's groups) the bits are equal; the DMA form also meets the
-    oracle bars. N 400 (ragged against the 128-row block), K with a 32-value tail for Q8_0."""
+def test_skinny_block_widths_agree(mx, monkeypatch, wtype, M):
+    """The skinny kernel's 64-wide blocks of four K ways against its 128-wide blocks of two on the same
+    packed activations (MI355X_SKINNY_BLOCKS, the blocks of one round, decides between them: 7 tiles of
+    64 fit 8, not 4): the same decoders and fp16 products, summed over K in another order, so they differ by
+    fp32 rounding only and are not the same launch; both meet the oracle bars. N 400 (ragged against
+    both widths), K with a 32-value tail for Q8_0."""
     import torch
     K = 1024 if wtype in SUPER_BLOCK else 1056
     N = 400
@@ -548,17 +546,21 @@ def test_skinny_dma_matches_register_kernel(mx, monkeypatch, wtype, M):
     w = mx.upload_weight(wtype, P, N, K)
     a16, sc = mx.pack_act(_dev(Xf))
     got = {}
-    for dma in ("1", "0"):
-        monkeypatch.setenv("MI355X_SKINNY_DMA", dma)
-        monkeypatch.setenv("MI355X_SKINNY_BLOCKS", "4")   # one K split: the whole K in each block
+    for blocks in ("8", "4"):
+        monkeypatch.setenv("MI355X_SKINNY_BLOCKS", blocks)
         c = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
         mx.gemm(wtype, a16, sc, K, [(w, N, 0, N, c)])
         torch.cuda.synchronize()
-        got[dma] = c.cpu().numpy()
-    assert np.isfinite(got["1"]).all()
-    assert np.array_equal(got["1"], got["0"]), float(np.abs(got["1"] - got["0"]).max())
-    _assert_bars(O.mul_mat(wtype, P, Xf, N, K), got["1"], M, N, f"skinny dma {O.TYPE_NAMES[wtype]} M={M}",
-                 cos_floor=0.999 if M >= 8 else -1.0)
+        got[blocks] = c.cpu().numpy()
+    assert np.isfinite(got["8"]).all() and np.isfinite(got["4"]).all()
+    # partial sums of up to K products stay below the row's sum of magnitudes: K 2^-24 of it bounds either order
+    mags = np.abs(Xf).astype(np.float64) @ np.abs(O.f16_bits_to_f32(O.dequantize_f16(wtype, P, K)).reshape(N, K)).T
+    assert (np.abs(got["8"] - got["4"]) <= 2 * K * 2.0 ** -24 * 1.01 * mags).all()
+    if M >= 32:
+        assert not np.array_equal(got["8"], got["4"]), "the same launch twice"
+    for c in got.values():
+        _assert_bars(O.mul_mat(wtype, P, Xf, N, K), c, M, N, f"skinny widths {O.TYPE_NAMES[wtype]} M={M}",
+                     cos_floor=0.999 if M >= 8 else -1.0)
 
 
 @pytest.mark.parametrize("wtype", SKINNY_TYPES)
