@@ -282,6 +282,10 @@ static double tile_fill(int64_t M, int64_t N, int bm) {
 //     where its tiles fill the chip (14336 x 4096 at M 512, 224 tiles: 0.93x) and loses 1.1-1.4x where
 //     the last round is mostly empty (at M 600, 280 tiles); Q8_0 past 2^26 weights, whose decode pass
 //     moves twice the bytes, only from M 768.
+//     Q8_0 up to 2^25 weights stays inside too where that launch makes one full round: up to 256 rows its
+//     K split, from K 4096 and 2^24 weights on (4096 x 4096 M 160 0.96x, 8192 x 4096 0.91x, 6144 x 5120 0.89x; not
+//     5632 x 4096, whose six splits are 264 blocks: 1.36x; 8192 x 2560 1.10x), and up to 767 its tiles where they
+//     take 0.85 of the chip (16384 x 1024 M 512 0.91x, 12800 x 2560 M 600 0.96x; 11008 x 2816 M 640, 0.84, 1.12x).
 // Panels under 2^22 weights keep lines drawn with the older fp16 GEMM: such calls are a few
 // microseconds of launches either way. Same fp16 weights and activations in both forms.
 static bool mul_mat_decode_first(int wtype, int64_t M, int64_t N, int64_t K) {
@@ -302,6 +306,15 @@ static bool mul_mat_decode_first(int wtype, int64_t M, int64_t N, int64_t K) {
         case mx::T_Q8_0:
             if (!panel) return M >= 1024 || (M >= 512 && K % 256 && N >= K);
             if (split) return M >= 768;
+            if (w25 && M < 768 && K % 256 == 0 && ((M <= 256 && K >= 4096 && w >= ((int64_t)1 << 24)) || tile_fill(M, N, 128) >= 0.85)) {
+                mx::GemmArgs a;
+                memset(&a, 0, sizeof(a));
+                a.M = (int)M;
+                a.K = (int)K;
+                a.ng = 1;
+                a.g[0].N = (int)N;
+                if (mx::gemm_one_round(wtype, a)) return false;
+            }
             if (w25 || M >= 768) return true;
             return M >= 384 && w26 && tile_fill(M, N, 128) < 0.8;
         default: return false;

@@ -2326,6 +2326,11 @@ static GemmPlan plan_gemm(int wt, const GemmArgs & a, int slabs) {
     return p;
 }
 
+bool gemm_one_round(int wt, const GemmArgs & a) {
+    const GemmPlan p = plan_gemm(wt, a, 64);
+    return !p.skinny && (int64_t)tiles_of(a, kCfgs[p.cfg].bm, kCfgs[p.cfg].bn) * p.ks <= cu_count();
+}
+
 size_t gemm_split_bytes(int wt, const GemmArgs & a) {
     const GemmPlan p = plan_gemm(wt, a, 64);
     return p.slabs ? (size_t)p.ks * (size_t)a.M * (size_t)total_cols(a) * sizeof(float) : 0;

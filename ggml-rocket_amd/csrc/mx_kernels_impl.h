@@ -136,6 +136,8 @@ hipError_t launch_gemm(int wt, const GemmArgs & a, int n_tiles_total, hipStream_
 // whether launch_gemm, with part_bytes of partial workspace, would add into its outputs (a
 // two-way K split) rather than write them
 bool gemm_accumulates(int wt, const GemmArgs & a, size_t part_bytes);
+// a tiled launch with its fastest K split has a CU for every block
+bool gemm_one_round(int wt, const GemmArgs & a);
 // partial workspace bytes of the launch's fastest K split (0 if it splits two ways or less)
 size_t gemm_split_bytes(int wt, const GemmArgs & a);
 hipError_t launch_dequant_f16(int wt, const void * W, int64_t rows, int64_t K, uint16_t * out, hipStream_t st);

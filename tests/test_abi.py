@@ -120,11 +120,10 @@ def test_mul_mat_id_regrouped_layout_limits():
 
 def test_mul_mat_workspace_sizes_the_decode_first_weight():
     """mi355x_mul_mat_workspace_for makes room for the tiled fp16 weight where the decode-first
-    form runs (Q6_K / Q5_K / MXFP4 at M >= 512; Q4_0 at M >= 1024, or at M >= 512 with N >= K;
-    Q8_0 at M >= 1024, and at M 512 only where N >= K, N * K > 2^24 and the all-DMA kernel's
-    128 x 256 tiles leave part of the chip idle, or with K off the 256-value blocks where N >= K)
-    and elsewhere sizes the pack and the in-GEMM decode's split partials only (host-side sizing:
-    no GPU needed)."""
+    form runs (never up to 128 rows; above, weights of 2^22 to 2^25 values, except Q8_0 where the launch
+    that decodes inside makes one full round, and Q4_K and Q8_0 with K split deep; larger weights and
+    smaller ones from the M of their type) and elsewhere sizes the pack and the in-GEMM decode's split
+    partials only (host-side sizing: no GPU needed)."""
     import ggml_mi355x as mx
     L = mx.lib()
     for wt, M, N, K, first in [(mx.Q6_K, 512, 1024, 3072, True), (mx.Q6_K, 128, 1024, 3072, False),
@@ -134,7 +133,12 @@ def test_mul_mat_workspace_sizes_the_decode_first_weight():
                                (mx.Q8_0, 1024, 1024, 3072, True), (mx.Q4_K, 2048, 1024, 3072, False),
                                (mx.Q4_K, 512, 6144, 4096, True), (mx.Q4_K, 512, 28672, 4096, False),
                                (mx.Q5_K, 512, 1024, 3072, True), (mx.MXFP4, 512, 1024, 3072, True),
-                               (mx.Q4_0, 512, 1024, 3072, False), (mx.Q4_0, 512, 3072, 1024, True)]:
+                               (mx.Q4_0, 512, 1024, 3072, False), (mx.Q4_0, 512, 3072, 1024, True),
+                               (mx.Q8_0, 160, 4096, 4096, False), (mx.Q8_0, 160, 5632, 4096, True),
+                               (mx.Q8_0, 256, 6144, 5120, False), (mx.Q8_0, 257, 4096, 4096, True),
+                               (mx.Q8_0, 160, 8192, 2560, True), (mx.Q8_0, 160, 3072, 3072, True),
+                               (mx.Q8_0, 512, 16384, 1024, False), (mx.Q8_0, 640, 11008, 2816, True),
+                               (mx.Q4_K, 160, 4096, 4096, True)]:
         pack = int(L.mi355x_mul_mat_workspace(M, K))
         poff = (pack + 255) // 256 * 256
         arr = (mx.GemmOut * 1)()
