@@ -533,7 +533,9 @@ static FaPlan fa_plan(const mi355x_fa_args * a, int nsplit_req) {
 
 // The fused MLA's launch arguments. KV split: a block takes about 2.9 us a key tile after some 12 us
 // of prologue (measured at 16 heads, 512 queries, n_kv 4096); a split writes its partial rows and
-// reads them back in the combine launch.
+// reads them back in the combine launch, which walks the splits in turn, at least 0.85 us each (16 heads, T 1-32: two
+// tiles a split instead of four gain 6 us at 4 splits, nothing at 16 and lose 6 at 32; whole call T 8 n_kv 512
+// with soft-cap and holes 36.0 -> 29.7).
 static mx::FaArgs fa_mla_lower(const mi355x_fa_args * a) {
     mx::FaArgs f = fa_lower(a, 1);
     f.D = 576;
@@ -542,9 +544,9 @@ static mx::FaArgs fa_mla_lower(const mi355x_fa_args * a) {
     const int64_t nb = mx::fa_mla_blocks(f);
     const double part_mb = (double)a->T * a->H * 512 * 8.0 / 1e6;
     double best = 0.0;
-    for (int ns = 1; ns <= std::min(std::max(ntiles / 4, 1), 64); ns++) {
+    for (int ns = 1; ns <= std::min(ntiles, 64); ns++) {
         const int64_t rounds = (nb * ns + cus - 1) / cus;
-        const double us = (double)rounds * (12.0 + ((ntiles + ns - 1) / ns) * 2.9) + (ns > 1 ? 3.0 + ns * part_mb / 6.0 : 0.0);
+        const double us = (double)rounds * (12.0 + ((ntiles + ns - 1) / ns) * 2.9) + (ns > 1 ? 3.0 + ns * std::max(0.85, part_mb / 6.0) : 0.0);
         if (ns == 1 || us < best - 1e-9) {
             best = us;
             f.nsplit = ns;

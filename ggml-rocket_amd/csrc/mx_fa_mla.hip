@@ -17,7 +17,9 @@
 // What bounds it: per tile 2176 clocks of MFMA a SIMD and 2480 of LDS traffic a CU (147 KB of K
 // fragments, 64 KB of V and 32 KB of P fragments, 74 KB of DMA), but also some 1500 clocks of softmax,
 // which one wave a SIMD cannot overlap with its MFMAs: 2.9 us a tile, 12 us of prologue and 7 us for a
-// split's partial rows. 64 rows a block because the O tile of 128 would leave no registers for Q; the key
+// split's partial rows. Three registers a lane spill, outside the loop over the tiles: a reload in it would wait
+// for the next tile's DMA, as a mixed tile's mask loads do (with ten spilled, T 512 n_kv 4096 took 160 us with
+// soft-cap, now 144; with a mask of holes in every tile 151, now 148). 64 rows a block because the O tile of 128 would leave no registers for Q; the key
 // range is split across blocks to fill the chip, partial rows merged by fa_combine. The older form
 // (fp16 Q and keys, transposed values, F32 scores through HBM, a softmax pass, two GEMMs) moved 134 MB of
 // scores and P out and back. Whole call, 16 heads on one KV head, causal (older -> this, us): T 512 n_kv
@@ -41,7 +43,8 @@ constexpr int ML_PER = ML_TILE / (ML_THREADS * 16);    // 18 DMA instructions pe
 constexpr int ML_P = 2 * ML_TILE;                      // P: [64 queries][64 keys] fp16
 constexpr int ML_MAX = ML_P + ML_BQ * ML_KT * 2;       // row maxima: [64 queries][2 key groups]
 constexpr int ML_SCALE = ML_MAX + ML_BQ * 8;           // Q row scales [64], then the range
-constexpr int ML_CLS = ML_SCALE + ML_BQ * 4 + 16;      // the block's class of every key tile
+constexpr int ML_TOK = ML_SCALE + ML_BQ * 4 + 16;      // mask row of each query row [64]
+constexpr int ML_CLS = ML_TOK + ML_BQ * 4;             // the block's class of every key tile
 constexpr int ML_MAX_TILES = FA_MLA_MAX_KV / ML_KT;
 constexpr int ML_LDS = ML_CLS + ML_MAX_TILES;
 static_assert(ML_PER * ML_THREADS * 16 == ML_TILE && ML_LDS <= 160 * 1024, "LDS");
@@ -107,7 +110,7 @@ enum : uint8_t { ML_SKIP = 0, ML_FULL = 1, ML_MIXED = 2 };   // the classes fa_p
 template <bool SOFTCAP>
 __global__ void __launch_bounds__(ML_THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) fa_mla_kernel(FaArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__   // the buffer resource type exists in the device pass only
-    extern __shared__ __align__(16) uint8_t smem[];
+    extern __shared__ __align__(64) uint8_t smem[];
     const int t = threadIdx.x, lane = t % WAVE, wave = __builtin_amdgcn_readfirstlane(t / WAVE);
     const int lc = lane % 16, lg = lane / 16;
     const int kg = wave / 2, qg = wave % 2;
@@ -232,14 +235,7 @@ __global__ void __launch_bounds__(ML_THREADS) __attribute__((amdgpu_waves_per_eu
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int s = 0; s < ML_Q1; s++) asm volatile("" : "+a"(qf[i][s]));
-    float qsc[2];
-    int mtok[2];   // the mask row
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int r = 32 * qg + 16 * i + lc;
-        qsc[i] = ((const float *)(smem + ML_SCALE))[r];
-        mtok[i] = min(r0 + r, rows - 1) / g;
-    }
+    if (t < ML_BQ) ((int *)(smem + ML_TOK))[t] = min(r0 + t, rows - 1) / g;   // the mask rows
     ml_barrier_lgkm();   // the second buffer is free
     if (nt > 1) {
         issue(1);
@@ -268,7 +264,6 @@ __global__ void __launch_bounds__(ML_THREADS) __attribute__((amdgpu_waves_per_eu
     const int vkey = 8 * lg + 4 * (vs / 8) + (vs / 4) % 2;   // h = 0; its swizzle (key / 2 % 8) is even, h = 1's one more
     const uint32_t smem_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)smem;
     const uint32_t vbase0 = smem_lds + vkey * ML_RB + 256 * wave + 16 * ((vs % 4) / 2) + 8 * (vs % 2);
-    const uint32_t vbase1 = smem_lds + (vkey + 2) * ML_RB + 256 * wave + 16 * ((vs % 4) / 2 ^ 1) + 8 * (vs % 2);
     const uint32_t vx = 16 * ((vkey >> 1) & 6);              // dim tile d sits (32 d) ^ vx bytes on
     // fragment reads at 32-deep step st: chunk 4 st + lg of a row, i.e. one of two lane offsets (st even,
     // odd) plus 128 bytes every two steps
@@ -336,13 +331,19 @@ __global__ void __launch_bounds__(ML_THREADS) __attribute__((amdgpu_waves_per_eu
             }
             // scores in units of log 2: s * f with f = Q's row scale * log2(e); softcap, mask and the key
             // bound, where the tile has them, work on the scaled score first
-            float f[2] = {qsc[0] * LOG2E, qsc[1] * LOG2E};
+            // (the row scales and mask rows come from LDS each time: held, they would spill, and a spill's
+            // reload waits for the K tile in flight)
+            float qsc[2], f[2];
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                qsc[q] = ((const float *)(smem + ML_SCALE))[32 * qg + 16 * q + lc];
+                f[q] = qsc[q] * LOG2E;
+            }
             const bool tail = j0 + ML_KT > a.KV;
             if (SOFTCAP || tail || (cls == ML_MIXED && a.mask)) {
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
-                    int tk = mtok[q];
-                    asm("" : "+v"(tk));   // the row's address is worked out here, not held across the loop
+                    const int tk = ((const int *)(smem + ML_TOK))[32 * qg + 16 * q + lc];
                     const uint16_t * mrow = a.mask + (int64_t)tk * a.mask_nb1;
 #pragma unroll
                     for (int k = 0; k < 2; k++) {
@@ -438,9 +439,9 @@ __global__ void __launch_bounds__(ML_THREADS) __attribute__((amdgpu_waves_per_eu
             half8 pf[4], vf[2][4];
             auto read_v = [&](int g) {
 #pragma unroll
-                for (int d = 0; d < 4; d++) {
+                for (int d = 0; d < 4; d++) {   // h = 1: two rows on, its chunk one over
                     const uint32_t x = ((32u * d) ^ vx) + (uint32_t)((i & 1) * ML_TILE + 32 * (g / 2) * ML_RB + 128 * (g % 2));
-                    const half4v lo = ml_tr_read(vbase0 + x), hi = ml_tr_read(vbase1 + x);
+                    const half4v lo = ml_tr_read(vbase0 + x), hi = ml_tr_read((vbase0 ^ 16) + x + 2 * ML_RB);
                     vf[g % 2][d] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                 }
             };

@@ -224,6 +224,9 @@ def test_flash_attn_mla_workspace_and_split():
     assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 1, 16, 4096))) == 16
     assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 512, 16, 64))) == 1
     assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 1, 16, 200000))) == 1   # past its class table
+    # short key ranges split down to two tiles, where the block's own time is the call's
+    assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 8, 16, 512))) == 4
+    assert L.mi355x_flash_attn_auto_split(ctypes.byref(args(k, 64, 16, 1024))) == 8
 
 
 def test_host_memory_matches_meminfo():
