@@ -1099,7 +1099,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(gemm_tf, 1), "peak": PEAK_F16_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(gemm_tf / PEAK_F16_TFLOPS, 4),
                      "traffic": traffic, "traffic_source": traffic_src,
-                     "kernel": ("gemm_f16_kernel / gemm_f16_cols_kernel (LDS-DMA, fp16 MFMA 32x32x16)" if args.route == "prepacked-q"
+                     "kernel": ("gemm_f16_1w_kernel (tiled fp16 weights, one wave a SIMD, LDS DMA, fp16 MFMA 16x16x32)" if args.route == "prepacked-q"
                                 else "gemm_kernel<Q4_K> (register-staged, Q4_K decoded into LDS, fp16 MFMA 32x32x16)"),
                      "avg_launch_us": round(gemm["sec"] / gemm["launches"] * 1e6, 2),
                      "flop_per_launch": round(gemm["flops"] / gemm["launches"])},

@@ -1013,7 +1013,8 @@ gemm_f16_cols_kernel(GemmArgs args) {
 // flight), one barrier, then buffer s % NS is refilled with stage s + NS. Past the last stage the
 // last one is fetched again into buffers nobody reads, so the wait counts are constants.
 // Rows past M or N read the last real row. The MFMA's first operand is the weight, so a lane holds
-// 4 consecutive output columns of one row and stores 16 bytes at once.
+// 4 consecutive output columns of one row and stores 16 bytes at once. The two widest tiles spill
+// outside the loop over the stages: 8 registers (256 x 224) and 74 (256 x 256) a lane, once per block.
 //
 // A launch of few tiles splits K args.ksplit ways (each split a slab of args.part, summed in split
 // order by reduce_splits_kernel). Measured against gemm_f16_kernel and its two-width variant on
@@ -1073,8 +1074,9 @@ gemm_f16_1w_kernel(GemmArgs args) {
     const int per = (nk_all + ks - 1) / ks, kb = split * per;
     const int nk = max(0, min(nk_all, kb + per) - kb);
 
-    // each operand's buffer starts at the tile's first 16-row block; a lane's offset in it stays
-    // below 16 * K * 32 bytes (the launcher keeps K under ONE_WAVE_MAX_K)
+    // each operand's buffer starts at the tile's first 16-row block; a lane's offset in it, the stage's
+    // included, stays below 17 * 32 * K bytes: 256 rows from a row0 inside a block touch 17 of them
+    // (the launcher keeps K under ONE_WAVE_MAX_K)
     constexpr int KSTEP = 1024;   // bytes of a row block one stage of K takes
     const int64_t a0 = tiled_index(m0, 0, K), b0 = tiled_index((row0 + n0) & ~(int64_t)15, 0, K);
     const char * abase = (const char *)(args.A + a0) + (int64_t)kb * KSTEP;
@@ -1194,7 +1196,7 @@ gemm_f16_1w_kernel(GemmArgs args) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) crow[n + e] = v[e];
         }
-        __builtin_amdgcn_sched_barrier(0);   // one row block's products at a time: no spills
+        __builtin_amdgcn_sched_barrier(0);   // one row block's products at a time: few spills (see above)
     }
 #endif
 }
@@ -1994,8 +1996,9 @@ static int q4k_split(const GemmArgs & a, int bm, int bn, int cap) {
     return (nsb + per - 1) / per;
 }
 
-// gemm_f16_1w_kernel addresses a tile's rows by 32-bit byte offsets (16 row blocks of 32 K bytes)
+// gemm_f16_1w_kernel addresses a tile's rows by 32-bit byte offsets (up to 17 row blocks of 32 K bytes)
 constexpr int ONE_WAVE_MAX_K = 1 << 21;
+static_assert(17LL * 32 * ONE_WAVE_MAX_K < 0x7FFFFFFF, "32-bit offsets");
 
 static bool cfg_fits(int c, int wt, int K) {
     const CfgDesc & d = kCfgs[c];
