@@ -997,7 +997,8 @@ gemm_f16_cols_kernel(GemmArgs args) {
 // the DMA writes (128 is the CU's limit), and all of them issue their reads and DMA in one burst
 // after each stage's barrier. Here a block is four waves, one per SIMD, so a wave has 512 registers
 // and takes up to 128 x 112 of the output (accumulators in AGPRs): a 256 x 224 tile reads 69 bytes
-// a clock. With no second wave to cover for it, the wave has to keep its own MFMAs issuing: stage
+// a clock at the full MFMA rate (39 beside the DMA's 20 at the 0.54 it reaches at 512 x 28672 x
+// 4096). With no second wave to cover for it, the wave has to keep its own MFMAs issuing: stage
 // s is multiplied from registers while stage s + 1's fragments are read and stage s + NS's DMA is
 // issued, one read or one DMA after each MFMA (a 16 x 16 x 32 MFMA takes 16 clocks, a read or a
 // DMA 4 to 8 of issue). Two things keep those gaps that short: buffer loads, whose source is a
@@ -1008,7 +1009,9 @@ gemm_f16_cols_kernel(GemmArgs args) {
 //
 // A stage is 32 values of K for the tile's BM + BN rows; LDS slot (row r, chunk p) of its 4 chunks a
 // row holds logical chunk p ^ ((r / 4) & 3), so the 16 rows of a fragment read fall on 16 distinct
-// bank groups. Per stage, after its first MFMA (whose operands are the wave's last reads of the
+// 16-byte slots of 256 bytes. SQ_LDS_BANK_CONFLICT still counts four cycles a read (none for the
+// 128-byte rows of gemm_f16_kernel), under the MFMAs: the waves wait on LDS 4-8% of their time. Per
+// stage, after its first MFMA (whose operands are the wave's last reads of the
 // stage's buffer): wait until stage s + 1 has landed (the (NS - 2) stages behind it may be in
 // flight), one barrier, then buffer s % NS is refilled with stage s + NS. Past the last stage the
 // last one is fetched again into buffers nobody reads, so the wait counts are constants.
