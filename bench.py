@@ -877,7 +877,7 @@ def configs_bench(args, subset=False, print_line=True):
     torch.cuda.empty_cache()
     # FLASH_ATTN_EXT with the absorbed MLA's head dims (DeepSeek-style: keys of 576, values the
     # first 512 of them), 16 query heads on one KV head, 512 queries over 4096 keys, causal: the
-    # two-GEMM path for head dims past 256
+    # fused kernel of that shape
     T, H, HK, D, DV, n_kv = 512, 16, 1, 576, 512, 4096
     q = torch.randn(T, H, D, device="cuda")
     kc = torch.randn(n_kv, HK, D, device="cuda").half()

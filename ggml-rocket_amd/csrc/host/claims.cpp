@@ -441,7 +441,7 @@ static bool claim_flash_attn(const mi355x_tensor * op) {
     if (!ref_rules) return false;
     // what the kernels read: head dims the fused kernel holds zero-padded (dk, dv <= 256; built
     // for 64/64, 128/128, the MLA 192/128 and 256/256) or, past those, the two-GEMM path (dk % 32
-    // == 0, dv % 8 == 0, both up to 1024: the absorbed MLA's 576 / 512); element strides;
+    // == 0, dv % 8 == 0, both up to 1024; the absorbed MLA's 576 / 512 fused); element strides;
     // 16-byte rows
     int dk_pad = 0, dv_pad = 0;
     const bool dims = (head_dim <= 256 && dv <= 256 && mx::fa_pad_dims((int)head_dim, (int)dv, dk_pad, dv_pad)) ||

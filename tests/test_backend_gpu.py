@@ -213,7 +213,7 @@ def test_flash_attn_mla_graph(be):
 def test_flash_attn_absorbed_mla_graph(be):
     """The absorbed MLA's FLASH_ATTN_EXT through graph_compute: keys of 576, values of 512 as a view
     of the keys' first 512 dims (the latent cache read twice), 16 query heads on one KV head, causal
-    at n_kv 1024; claimed and run on the device (the two-GEMM path), no CPU fallback."""
+    at n_kv 1024; claimed and run on the device (the fused kernel), no CPU fallback."""
     D, DV, T, H, KV, HK = 576, 512, 96, 16, 1024, 1
     Q = O.fill_normal((H, T, D), 970)
     K16 = O.f32_to_f16_bits(O.fill_normal((HK, KV, D), 971))

@@ -226,7 +226,7 @@ def test_mul_mat_quant_sweep(mx, K, N, M, wtype):
                                          # 32 / 128-row tiles (N % 16 == 0, as every MUL_MAT here takes)
                                          (O.Q6_K, 520, 112, 256), (O.Q8_0, 530, 208, 192)])
 def test_mul_mat_decode_first(mx, wtype, M, N, K):
-    """Q6_K / Q5_K / MXFP4 / Q8_0 / Q4_0 / Q4_K at M >= 512: with mi355x_mul_mat_workspace_for bytes the weight is decoded once
+    """Q6_K / Q5_K / MXFP4 / Q8_0 / Q4_0 / Q4_K where the decode-first form is chosen: with mi355x_mul_mat_workspace_for bytes the weight is decoded once
     into tiled fp16 in the workspace and multiplied by the fp16 GEMM; with only the pack's bytes it
     is decoded inside the GEMM. Both forms meet the oracle's bars and agree with each other to
     fp32 summation order (same fp16 weights and activations)."""

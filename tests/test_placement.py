@@ -75,7 +75,7 @@ CASES = [
     ("FA: dk 128 / dv 64 -> offload (dv padded to 128)", True, lambda: fa_supported(128, 256, 8, 1024, 2, mx.F16, 0.0, 0, 64)),
     ("FA: dk 192 / dv 192 -> offload (padded to 256)", True, lambda: fa_supported(192, 256, 8, 1024, 2, mx.F16, 0.0)),
     ("FA: head_dim 256 (Gemma) -> offload", True, lambda: fa_supported(256, 256, 8, 1024, 2, mx.F16, 0.0)),
-    ("FA: dk 576 / dv 512 (absorbed MLA) -> offload (two-GEMM path)", True, lambda: fa_supported(576, 256, 8, 1024, 1, mx.F16, 0.0, 0, 512)),
+    ("FA: dk 576 / dv 512 (absorbed MLA) -> offload", True, lambda: fa_supported(576, 256, 8, 1024, 1, mx.F16, 0.0, 0, 512)),
     ("FA: head_dim 288 -> offload (two-GEMM path)", True, lambda: fa_supported(288, 256, 8, 1024, 2, mx.F16, 0.0)),
     ("FA: head_dim 1056 -> CPU (> 1024)", False, lambda: fa_supported(1056, 256, 8, 1024, 2, mx.F16, 0.0)),
     # Narrower: a quantized type without a device decoder is declined (the reference takes any
